@@ -11,28 +11,31 @@
 //
 // Rays are re-walked from the ray set-up (nothing per sample is stored); the
 // scatter of weight * trilinear weight is bound by the line requests of
-// device atomics, so each family of rays has its own way to need fewer:
-//   * primary rays: the 64 rays of a wave march side by side, so
-//     a wave adds a chunk of up to 16 steps into an LDS window over the
-//     texels they touch there (float64: LDS float32 adds run a lane at a
-//     time, ~200 cycles per wave instruction against ~11) and flushes the
-//     window with one atomic per texel, rows of texels together;
-//   * shadow rays and LAO taps start at surfaces of different depths, so
-//     their samples share little: each goes to a corner-packed accumulator of 8 floats per
+// device atomics, and there are two ways to need fewer:
+//   * cells: each sample goes to a corner-packed accumulator of 8 floats per
 //     cell (the cell layout of the density: cell (i,j,k) for i,j,k in
 //     [-1, n-1] holds texels i..i+1 x j..j+1 x k..k+1), 8 lanes adding the 8
 //     corners of one sample in one 32-byte request, and neighbouring rays of
 //     a pixel row in one cell add once.  A gather pass folds the cells into
-//     the texel gradient.
-// Measured at 128^3 / 512^2 / 256 steps: 0.35 ms with the primary rays in the
-// cells too, 0.27 so (0.45 with the LAO taps in windows: each of their
-// surfaces needs a window of its own).  Parameter gradients are reduced per
-// block, then one atomic each.
+//     the texel gradient;
+//   * windows, for primary rays: the 64 rays of a wave march side by side, so
+//     a wave adds a chunk of up to 16 steps into an LDS window over the
+//     texels they touch there (float64: LDS float32 adds run a lane at a
+//     time, ~200 cycles per wave instruction against ~11) and flushes the
+//     window with one atomic per texel, rows of texels together.
+// Windows pay only while the rays of a wave are close in texels and not all
+// in one (window_scatter): at 128^3 / 512^2 / 256 steps 0.25 ms against 0.32
+// in cells, at 128^2 pixels 0.87 against 0.25.  Shadow rays and LAO taps start at
+// surfaces of different depths, so their samples share little and go to the
+// cells (0.45 ms with the LAO taps in windows: each of their surfaces needs a
+// window of its own).  Parameter gradients are reduced per block, then one
+// atomic each.
 #include "march.hpp"
 
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 namespace vkhr {
@@ -69,7 +72,7 @@ __device__ __forceinline__ bool in_range(const RaymarchArgs& f, const double x[3
 // (measured, us of the adjoint: 512 texels 361, 768 277, 1264 280, 1728 267,
 // 2500 272).
 constexpr int kWindow = 1728, kWindowSide = 12;
-struct ScatterLds {
+struct WindowLds {
     double window[kWindow];
 };
 
@@ -133,7 +136,7 @@ __device__ __forceinline__ void window_add(const Window& win, const RaymarchArgs
 // an axis), and flushes each window into the gradient.  Every lane of the
 // wave calls it.
 template <class Add>
-__device__ __forceinline__ void scatter_windows(const AdjointArgs& a, ScatterLds& lds, bool active, const int lo[3],
+__device__ __forceinline__ void scatter_windows(const AdjointArgs& a, WindowLds& lds, bool active, const int lo[3],
                                                 const int hi[3], Add add) {
     const int lane = __lane_id();
     unsigned long long rest = __ballot(active);
@@ -188,7 +191,7 @@ __device__ __forceinline__ void scatter_windows(const AdjointArgs& a, ScatterLds
 // sample parameters t of the shader's float loop, samples [0, n) of each
 // active lane's ray, weight c per sample.  The loop runs to the wave's
 // longest ray so that every lane takes part in the windows.
-__device__ void scatter_rays(const AdjointArgs& a, ScatterLds& lds, bool active, const double x0[3], const double dx[3],
+__device__ void scatter_rays(const AdjointArgs& a, WindowLds& lds, bool active, const double x0[3], const double dx[3],
                              int n, float c) {
     const RaymarchArgs& f = a.f;
     const float step = f.step_size;
@@ -246,7 +249,7 @@ struct CellLds {
     float w[8][kWave];
 };
 
-static_assert(sizeof(CellLds) <= sizeof(ScatterLds), "the wave's LDS holds either");
+static_assert(sizeof(CellLds) <= sizeof(WindowLds), "the wave's LDS holds either");
 
 // Adds c * (trilinear corner weights) of every lane's sample to the cell
 // accumulator; lanes without a sample pass cell == kNoCell.  The samples
@@ -363,7 +366,9 @@ gather_cells_kernel(const float* __restrict__ cg, const float* __restrict__ texe
             for (int r = 0; r < kFoldRows; ++r) {
                 if (x >= nx || y0 + r >= ny) continue;
                 const size_t i = size_t(x) + size_t(nx) * (size_t(y0 + r) + size_t(ny) * size_t(z - 1));
-                grad[i] += texels[size_t(x) + cx * (size_t(y0 + r) + cy * size_t(z - 1))] + below[r];
+                float sum = below[r];
+                if (texels) sum += texels[size_t(x) + cx * (size_t(y0 + r) + cy * size_t(z - 1))];
+                grad[i] += sum;
             }
         }
 #pragma unroll
@@ -374,24 +379,28 @@ gather_cells_kernel(const float* __restrict__ cg, const float* __restrict__ texe
     }
 }
 
-// Which walk adjoint_tile takes: the primary rays with the parameter gradients
-// (and the loss), or the shadow rays with the LAO taps.
-enum AdjointWalk { kWalkPrimary, kWalkShadow };
+// What adjoint_tile takes: the primary rays with the parameter gradients (and
+// the loss) and nothing else, or the shadow rays, the LAO taps or both.
+enum AdjointWalk { kWalkPrimary = 1, kWalkShadow = 2, kWalkOcclusion = 4 };
 
 // The adjoint of one pixel (volume.frag:31-102 differentiated).  Called by
 // all 256 threads of a block: 2x2 waves of 8x8 pixels from (x0, y0); red is
-// the block's reduction buffer for the parameter gradients.
+// the block's reduction buffer for the parameter gradients.  Lds: WindowLds
+// when the primary rays go through windows, else CellLds.
+template <class Lds>
 __device__ __forceinline__ void adjoint_tile(const AdjointArgs& a, int x0, int y0, double (*red)[256 / kWave],
-                                             ScatterLds* scatter, AdjointWalk walks) {
+                                             Lds* scatter, int walks) {
     // red: 4 x (waves per block) doubles
+    constexpr bool kWindows = std::is_same<Lds, WindowLds>::value;
     const RaymarchArgs& f = a.f;
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    ScatterLds& L = scatter[wave];
-    // the primary walk spreads a wave over the whole tile (lanes two pixels
+    Lds& L = scatter[wave];
+    CellLds& cells = *reinterpret_cast<CellLds*>(&L);
+    // the windows' walk spreads a wave over the whole tile (lanes two pixels
     // apart): rays in one cell would add to the same LDS words in turn
-    const bool primary = walks == kWalkPrimary;
-    const int px = primary ? x0 + (wave & 1) + 2 * (lane & 7) : x0 + (wave & 1) * 8 + (lane & 7);
-    const int py = primary ? y0 + (wave >> 1) + 2 * (lane >> 3) : y0 + (wave >> 1) * 8 + (lane >> 3);
+    const bool primary = walks == kWalkPrimary, spread = kWindows && primary;
+    const int px = spread ? x0 + (wave & 1) + 2 * (lane & 7) : x0 + (wave & 1) * 8 + (lane & 7);
+    const int py = spread ? y0 + (wave >> 1) + 2 * (lane >> 3) : y0 + (wave >> 1) * 8 + (lane >> 3);
     const bool inside = px < f.width && py < f.height;
     const size_t pix = inside ? size_t(py) * f.width + px : 0;
 
@@ -460,7 +469,12 @@ __device__ __forceinline__ void adjoint_tile(const AdjointArgs& a, int x0, int y
         __syncthreads();  // red is reused by the next tile of a persistent block
 
         const Ray ray = setup_ray(f, px, py, inside && frag && c_primary != 0.0);
-        scatter_rays(a, L, ray.hit && c_primary != 0.0, ray.xs, ray.dx, frag ? r.n_primary : 0, float(c_primary));
+        const bool walk = ray.hit && c_primary != 0.0;
+        const int n = frag ? r.n_primary : 0;
+        if constexpr (kWindows)
+            scatter_rays(a, L, walk, ray.xs, ray.dx, n, float(c_primary));
+        else
+            scatter_rays_cells(a, cells, walk, ray.xs, ray.dx, n, float(c_primary));
         return;
     }
     // shadow rays: from the surface point to the light origin, every sample
@@ -469,16 +483,19 @@ __device__ __forceinline__ void adjoint_tile(const AdjointArgs& a, int x0, int y
         s[0] = r.sx; s[1] = r.sy; s[2] = r.sz;
         for (int k = 0; k < 3; ++k) sl[k] = a.light_texel[k] - s[k];
     }
-    // samples past the volume's support carry no gradient: the walk stops
-    // there (an upper bound on their count is enough, in_range does the rest)
-    int n_shadow = 0;
-    if (frag) {
-        double lo, hi;
-        support_interval(f, s, sl, &lo, &hi);
-        if (hi >= 0.0 && lo <= hi) n_shadow = min(a.n_steps, int(fmin(hi, 2.0) / double(f.step_size) * 1.0001) + 2);
+    if (walks & kWalkShadow) {
+        // samples past the volume's support carry no gradient: the walk stops
+        // there (an upper bound on their count is enough, in_range does the rest)
+        int n_shadow = 0;
+        if (frag) {
+            double lo, hi;
+            support_interval(f, s, sl, &lo, &hi);
+            if (hi >= 0.0 && lo <= hi)
+                n_shadow = min(a.n_steps, int(fmin(hi, 2.0) / double(f.step_size) * 1.0001) + 2);
+        }
+        scatter_rays_cells(a, cells, frag && adsm_on && c_shadow != 0.0, s, sl, n_shadow, float(c_shadow));
     }
-    CellLds& cells = *reinterpret_cast<CellLds*>(&L);
-    scatter_rays_cells(a, cells, frag && adsm_on && c_shadow != 0.0, s, sl, n_shadow, float(c_shadow));
+    if (!(walks & kWalkOcclusion)) return;
     // LAO taps: d ln(lao)/dD = -e / (8 - D), through min(v, clamp)
     const bool lao = frag && lao_on && G != 0.0;
     double v[8], D = 0.0;
@@ -503,17 +520,33 @@ __device__ __forceinline__ void adjoint_tile(const AdjointArgs& a, int x0, int y
     }
 }
 
-// blockIdx.z: 0 the primary rays and parameters, 1 the shadow rays and LAO.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
-adjoint_kernel(AdjointArgs) {
-    const AdjointArgs& a = kernel_args<AdjointArgs>();
+// blockIdx.z: 0 the primary rays and parameters, 1 the shadow rays, 2 the LAO
+// taps (with windows 1 both).  In workgroups of their own the taps wait for neither
+// walk: 64^3 / 24^2 / 16 steps 52 us against 67 behind the primary rays, 128^3 /
+// 300^2 / 300 steps 289 against 302.
+template <class Lds>
+__device__ __forceinline__ void adjoint_block(const AdjointArgs& a) {
     __shared__ double red[4][256 / kWave];
-    __shared__ ScatterLds scatter[256 / kWave];
+    __shared__ Lds scatter[256 / kWave];
     const int x0 = int(blockIdx.x) * 16, y0 = int(blockIdx.y) * 16;
     if (blockIdx.z == 0)
         adjoint_tile(a, x0, y0, red, scatter, kWalkPrimary);
-    else
+    else if (std::is_same<Lds, WindowLds>::value)
+        adjoint_tile(a, x0, y0, red, scatter, kWalkShadow | kWalkOcclusion);
+    else if (blockIdx.z == 1)
         adjoint_tile(a, x0, y0, red, scatter, kWalkShadow);
+    else
+        adjoint_tile(a, x0, y0, red, scatter, kWalkOcclusion);
+}
+
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+adjoint_windows_kernel(AdjointArgs) {
+    adjoint_block<WindowLds>(kernel_args<AdjointArgs>());
+}
+
+__global__ void __launch_bounds__(256)
+adjoint_cells_kernel(AdjointArgs) {
+    adjoint_block<CellLds>(kernel_args<AdjointArgs>());
 }
 
 // ---------------------------------------------------------- batched form
@@ -539,6 +572,8 @@ struct AdjointBatchDevice {
     AdjointChunk* clear_chunks;
     AdjointChunk* fold_chunks;
     float** losses;             // per render, nullable entries
+    uint32_t* order;            // the renders whose primary rays go through windows, then the others
+    uint32_t n_windows;
     uint32_t n_styles, n_renders;
     uint32_t n_clear_chunks, n_fold_chunks;
     uint32_t tiles_x, tiles_per_render;
@@ -576,15 +611,29 @@ adjoint_batch_forward_kernel(AdjointBatchDevice d, const AdjointArgs* __restrict
     raymarch_pixel<true>(args[r].f, px, py, OccupancyView{occ_lds, false});
 }
 
-// One block per (render, 16x16 tile): the adjoint with the L2 loss gradient.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
-adjoint_batch_backward_kernel(AdjointBatchDevice d, const AdjointArgs* __restrict__ args) {
+// One block per (render, 16x16 tile), the renders from order[first] on: the
+// adjoint with the L2 loss gradient.
+template <class Lds>
+__device__ __forceinline__ void adjoint_batch_block(const AdjointBatchDevice& d, const AdjointArgs* __restrict__ args,
+                                                    uint32_t first) {
     __shared__ double red[4][256 / kWave];
-    __shared__ ScatterLds scatter[256 / kWave];
+    __shared__ Lds scatter[256 / kWave];
     const uint32_t item = uint32_t(__builtin_amdgcn_readfirstlane(int(blockIdx.x)));
-    const uint32_t r = item / d.tiles_per_render, tile = item % d.tiles_per_render;
-    adjoint_tile(args[r], int(tile % d.tiles_x) * 16, int(tile / d.tiles_x) * 16, red, scatter, kWalkPrimary);
-    adjoint_tile(args[r], int(tile % d.tiles_x) * 16, int(tile / d.tiles_x) * 16, red, scatter, kWalkShadow);
+    const AdjointArgs& a = args[d.order[first + item / d.tiles_per_render]];
+    const uint32_t tile = item % d.tiles_per_render;
+    const int x0 = int(tile % d.tiles_x) * 16, y0 = int(tile / d.tiles_x) * 16;
+    adjoint_tile(a, x0, y0, red, scatter, kWalkPrimary);
+    adjoint_tile(a, x0, y0, red, scatter, kWalkShadow | kWalkOcclusion);
+}
+
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+adjoint_batch_windows_kernel(AdjointBatchDevice d, const AdjointArgs* __restrict__ args) {
+    adjoint_batch_block<WindowLds>(d, args, 0u);
+}
+
+__global__ void __launch_bounds__(256)
+adjoint_batch_cells_kernel(AdjointBatchDevice d, const AdjointArgs* __restrict__ args) {
+    adjoint_batch_block<CellLds>(d, args, d.n_windows);
 }
 
 // d_density += the fold of each style's cells.
@@ -629,6 +678,29 @@ static int diff_args(const vkhr_volume* volume, const vkhr_camera* camera, const
         a->shininess = diff->shininess;
     }
     return VKHR_OK;
+}
+
+// Whether the primary rays' samples go through windows: when a wave's rays
+// share texels but not one texel, and its chunk of steps fits a window.  The
+// pitch of the pixels and the step are in texels (of the mean side, at the
+// volume's centre); 16 pixels span a wave.  Measured (us of the adjoint, cells
+// / windows; hair, steps in brackets): pitch 0.036 (0.22) 331 / 436, 0.08
+// (0.45) 211 / 171, 0.23 (0.45) 140 / 97 at 64^3, 0.36 (0.9) 316 / 251 at
+// 128^3; 0.58 (0.9) 269 / 600, 1.4 (0.9) 215 / 730, 2.8 (3.6) 107 / 1000.
+static bool window_scatter(const RaymarchArgs& f, const vkhr_camera& camera) {
+    double away2 = 0.0, texels = 1.0, volume = 1.0;
+    for (int c = 0; c < 3; ++c) {
+        const double d = f.origin[c] + 0.5 * f.size[c] - f.eye[c];
+        away2 += d * d;
+        volume *= f.size[c];
+        texels *= f.nres[c];
+    }
+    const double texel = std::cbrt(volume / texels);
+    const double focal = std::sqrt(std::fabs(double(camera.projection[0]) * double(camera.projection[5])));
+    const double pitch = 2.0 * std::sqrt(away2 / (double(f.width) * f.height)) / (focal * texel);
+    const double step = double(f.radius) * double(f.step_size) / texel;
+    const double across = 16.0 * pitch + 2.0, along = std::fmin(16.0 * step, 8.0) + 2.0;
+    return pitch >= 0.18 && step <= 1.2 && across * across * along <= 850.0;
 }
 
 // The per-launch constants of the adjoint derived from the forward's.
@@ -681,9 +753,10 @@ extern "C" int vkhr_raymarch_adjoint(const vkhr_volume* volume, const vkhr_camer
     a->d_rgba = reinterpret_cast<const float4*>(d_rgba);
     a->d_params = d_params;
     finish_adjoint_args(a);
-    // the cells, then the texels (in the cells' pitch)
+    const bool windows = window_scatter(a->f, *camera);
+    // the cells, then with windows the texels (in the cells' pitch)
     const size_t n_cells = (size_t(volume->nx) + 1) * (size_t(volume->ny) + 1) * (size_t(volume->nz) + 1);
-    const size_t sums = (n_cells * 9 + 1) / 2 * 2, words = sums + 8;   // and the parameter sums
+    const size_t sums = (n_cells * (windows ? 9 : 8) + 1) / 2 * 2, words = sums + 8;   // and the parameter sums
     void* cg = nullptr;
     hipStream_t st = as_stream(stream);
     if ((rc = stream_scratch(words * sizeof(float), st, &cg))) {
@@ -691,7 +764,7 @@ extern "C" int vkhr_raymarch_adjoint(const vkhr_volume* volume, const vkhr_camer
         return rc;
     }
     a->cell_grad = static_cast<float*>(cg);
-    a->texel_grad = a->cell_grad + n_cells * 8;
+    a->texel_grad = windows ? a->cell_grad + n_cells * 8 : nullptr;
     a->param_sums = reinterpret_cast<double*>(a->cell_grad + sums);
     a->texel_row = size_t(volume->nx) + 1;
     a->texel_slice = a->texel_row * (size_t(volume->ny) + 1);
@@ -699,10 +772,12 @@ extern "C" int vkhr_raymarch_adjoint(const vkhr_volume* volume, const vkhr_camer
         delete a;
         return rc;
     }
-    // each walk family in workgroups of its own: z = 0 the primary rays
-    // (with LAO and parameters), z = 1 the shadow rays
-    dim3 grid((width + 15) / 16, (height + 15) / 16, 2);
-    adjoint_kernel<<<grid, 256, 0, st>>>(*a);
+    // each walk family in workgroups of its own
+    dim3 grid((width + 15) / 16, (height + 15) / 16, windows ? 2 : 3);
+    if (windows)
+        adjoint_windows_kernel<<<grid, 256, 0, st>>>(*a);
+    else
+        adjoint_cells_kernel<<<grid, 256, 0, st>>>(*a);
     const dim3 fold((volume->nx + kWave - 1) / kWave,
                     (volume->ny + kFoldRows * (256 / kWave) - 1) / (kFoldRows * (256 / kWave)),
                     (volume->nz + kFoldLevels - 1) / kFoldLevels);
@@ -765,6 +840,7 @@ int build_adjoint_batch(vkhr_adjoint_batch* b, const vkhr_adjoint_style* styles,
     }
     std::vector<AdjointArgs> args(n_renders);
     std::vector<float*> losses(n_renders, nullptr);
+    std::vector<uint32_t> order, in_cells;
     for (uint32_t r = 0; r < n_renders; ++r) {
         const vkhr_adjoint_render& in = renders[r];
         VKHR_REQUIRE(in.style < n_styles, VKHR_ERR_INVALID, "render %u: style %u of %u", r, in.style, n_styles);
@@ -786,14 +862,18 @@ int build_adjoint_batch(vkhr_adjoint_batch* b, const vkhr_adjoint_style* styles,
         a.texel_slice = size_t(a.f.nx) * a.f.ny;
         finish_adjoint_args(&a);
         losses[r] = in.loss;
+        (window_scatter(a.f, in.camera) ? order : in_cells).push_back(r);
     }
+    const uint32_t n_windows = uint32_t(order.size());
+    order.insert(order.end(), in_cells.begin(), in_cells.end());
     AdjointBatchDevice& d = b->d;
     if ((rc = upload_table(b, st, &d.styles)) || (rc = upload_table(b, clear, &d.clear_chunks)) ||
         (rc = upload_table(b, fold, &d.fold_chunks)) || (rc = upload_table(b, losses, &d.losses)) ||
-        (rc = upload_table(b, args, &b->args)))
+        (rc = upload_table(b, args, &b->args)) || (rc = upload_table(b, order, &d.order)))
         return rc;
     d.n_styles = n_styles;
     d.n_renders = n_renders;
+    d.n_windows = n_windows;
     d.n_clear_chunks = uint32_t(clear.size());
     d.n_fold_chunks = uint32_t(fold.size());
     d.tiles_x = (width + 15) / 16;
@@ -834,7 +914,9 @@ extern "C" int vkhr_adjoint_batch_launch(vkhr_adjoint_batch* b, vkhr_stream stre
         VKHR_CHECK_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
         adjoint_batch_clear_kernel<<<4096, 256, 0, s>>>(b->d);
         adjoint_batch_forward_kernel<<<b->n_items, 256, 0, s>>>(b->d, b->args);
-        adjoint_batch_backward_kernel<<<b->n_items, 256, 0, s>>>(b->d, b->args);
+        const uint32_t in_windows = b->d.n_windows * b->d.tiles_per_render, in_cells = b->n_items - in_windows;
+        if (in_windows) adjoint_batch_windows_kernel<<<in_windows, 256, 0, s>>>(b->d, b->args);
+        if (in_cells) adjoint_batch_cells_kernel<<<in_cells, 256, 0, s>>>(b->d, b->args);
         adjoint_batch_fold_kernel<<<4096, 256, 0, s>>>(b->d);
         hipError_t e = hipStreamEndCapture(s, &b->graph);
         VKHR_CHECK_HIP(e);
