@@ -65,6 +65,13 @@ unpack_counts_kernel(const long long* __restrict__ acc, uint32_t* __restrict__ c
 constexpr uint32_t kBinBricks = 8192;          // a histogram in 32 KB of LDS: up to 160^3
 constexpr uint32_t kBinBlocks = 256;           // rows of the histogram at most
 constexpr int kBinThreads = 1024, kBrickThreads = 256;
+// A workgroup adds at most this many entries: the further parts of a fuller
+// brick are workgroups of their own, which add to the zeroed voxels of the
+// brick with device atomics.  Without parts a million vertices in one brick
+// take 1.3 ms (the atomics alone 0.38), so 0.06; 1.77M in a sixteenth of a
+// 128^3 box 75 us, with parts of 2048 96, of 8192 73, but then 273k 56 instead
+// of 51.
+constexpr uint32_t kPartEntries = 4096;
 // Below this many vertices the launches outweigh the atomics in a small
 // volume: 64^3 at 200k vertices 19.7 us against 17.5, at 300k 19.8 against
 // 21.9 (128^3: 25.2 against 32.5 and 27.3 against 36.9).
@@ -80,8 +87,28 @@ struct VertexBins {
     uint32_t* hist;                  // blocks x n_bricks: counts, then the vertices of the blocks before
     uint32_t* total;                 // per brick
     uint32_t* start;                 // n_bricks + 1: the bricks' first entries
+    uint32_t* more;                  // n_bricks + 1: the further parts of the bricks before
+    uint32_t more_blocks;            // further parts at most
     unsigned long long* entries;     // local voxel (9 bits) and tangent (18 bits per component)
+    uint32_t* counts;                // nullable
+    uint4* acc;
 };
+
+// The parts of a brick past its first.
+__device__ __forceinline__ uint32_t further_parts(uint32_t entries) {
+    return entries > kPartEntries ? (entries - 1u) / kPartEntries : 0u;
+}
+
+// Calls voxel(i, v) for the brick's voxels inside the volume: i in the brick
+// (a thread's 512 / kThreads of them), v in the volume.
+template <int kThreads, typename Voxel>
+__device__ __forceinline__ void brick_voxels(const VertexBins& a, uint32_t brick, Voxel voxel) {
+    const uint32_t ox = 8u * (brick % a.bx), oy = 8u * (brick / a.bx % a.by), oz = 8u * (brick / (a.bx * a.by));
+    for (uint32_t i = threadIdx.x; i < 512u; i += kThreads) {
+        const uint32_t x = ox + (i & 7u), y = oy + ((i >> 3) & 7u), z = oz + (i >> 6);
+        if (x < a.g.nx && y < a.g.ny && z < a.g.nz) voxel(i, x + size_t(a.g.nx) * (y + size_t(a.g.ny) * z));
+    }
+}
 
 __device__ __forceinline__ uint32_t vertex_brick(const VertexBins& a, uint3 c) {
     return (c.x >> 3) + a.bx * ((c.y >> 3) + a.by * (c.z >> 3));
@@ -127,36 +154,51 @@ __global__ void __launch_bounds__(kBinThreads) vertex_columns_kernel(VertexBins 
     }
 }
 
-// Every block scans the bricks' totals for itself, which saves a launch.
+// Every block scans the bricks' totals for itself, which saves a launch
+// (entries in the low half of the words, further parts in the high one).
 __global__ void __launch_bounds__(kBinThreads) vertex_fill_kernel(VertexBins a) {
     extern __shared__ uint32_t cursor[];
-    __shared__ uint32_t wave_sums[kBinThreads / kWave];
+    __shared__ unsigned long long wave_sums[kBinThreads / kWave];
+    // the block's share of the bricks in parts (a vertex chunk is under two of n / kBinBlocks: half as many blocks at least)
+    __shared__ uint32_t parted[2u * kBinBricks / kBinBlocks], n_parted;
     constexpr uint32_t kPer = kBinBricks / kBinThreads;
+    if (threadIdx.x == 0) n_parted = 0u;
     const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     for (uint32_t i = threadIdx.x; i < a.n_bricks; i += kBinThreads) cursor[i] = a.total[i];
     __syncthreads();
     const uint32_t per = (a.n_bricks + kBinThreads - 1u) / kBinThreads, i0 = threadIdx.x * per;
-    uint32_t v[kPer], sum = 0;
+    uint32_t v[kPer];
+    unsigned long long sum = 0;
 #pragma unroll
     for (uint32_t c = 0; c < kPer; ++c) {
         v[c] = c < per && i0 + c < a.n_bricks ? cursor[i0 + c] : 0u;
-        sum += v[c];
+        sum += v[c] | (unsigned long long)(further_parts(v[c])) << 32;
     }
-    uint32_t scan = sum;
+    unsigned long long scan = sum;
     for (int o = 1; o < kWave; o <<= 1) {
-        const uint32_t below = __shfl_up(scan, o, kWave);
-        scan += int(lane) >= o ? below : 0u;
+        const unsigned long long below = __shfl_up(scan, o, kWave);
+        scan += int(lane) >= o ? below : 0ull;
     }
     if (lane == kWave - 1) wave_sums[wave] = scan;
     __syncthreads();
-    uint32_t at = scan - sum;
+    unsigned long long at = scan - sum;
     for (uint32_t w = 0; w < wave; ++w) at += wave_sums[w];
 #pragma unroll
     for (uint32_t c = 0; c < kPer; ++c) {
-        if (c < per && i0 + c < a.n_bricks) cursor[i0 + c] = at;
-        at += v[c];
+        if (c < per && i0 + c < a.n_bricks) {
+            cursor[i0 + c] = uint32_t(at);
+            if (blockIdx.x == 0) a.more[i0 + c] = uint32_t(at >> 32);
+            if (further_parts(v[c]) != 0u && (i0 + c) % gridDim.x == blockIdx.x) parted[atomicAdd(&n_parted, 1u)] = i0 + c;
+        }
+        at += v[c] | (unsigned long long)(further_parts(v[c])) << 32;
     }
+    if (blockIdx.x == 0 && threadIdx.x == kBinThreads - 1u) a.more[a.n_bricks] = uint32_t(at >> 32);
     __syncthreads();
+    for (uint32_t b = 0; b < n_parted; ++b)
+        brick_voxels<kBinThreads>(a, parted[b], [&](uint32_t, size_t voxel) {
+            a.acc[voxel] = make_uint4(0u, 0u, 0u, 0u);
+            if (a.counts) a.counts[voxel] = 0u;
+        });
     const uint32_t* row = a.hist + size_t(blockIdx.x) * a.n_bricks;
     for (uint32_t i = threadIdx.x; i < a.n_bricks; i += kBinThreads) {
         if (blockIdx.x == 0) a.start[i] = cursor[i];
@@ -177,15 +219,31 @@ __global__ void __launch_bounds__(kBinThreads) vertex_fill_kernel(VertexBins a) 
     }
 }
 
-// One brick per workgroup.
-__global__ void __launch_bounds__(kBrickThreads)
-vertex_brick_kernel(VertexBins a, uint32_t* __restrict__ counts, uint4* __restrict__ acc) {
+// One part of a brick per workgroup: the further parts, then the first ones.
+__global__ void __launch_bounds__(kBrickThreads) vertex_brick_kernel(VertexBins a) {
     __shared__ unsigned long long words[512][2];
-    const uint32_t brick = blockIdx.x, first = a.start[brick], end = a.start[brick + 1u];
+    __shared__ uint32_t group, found;
+    uint32_t brick = blockIdx.x - a.more_blocks, part = 0u;
+    if (blockIdx.x < a.more_blocks) {   // workgroup-uniform
+        if (blockIdx.x >= a.more[a.n_bricks]) return;
+        // the brick whose further parts hold this one: a group of bricks per thread, then a brick
+        const uint32_t per = (a.n_bricks + kBrickThreads - 1u) / kBrickThreads;
+        const uint32_t i = threadIdx.x * per;
+        if (i < a.n_bricks && a.more[i] <= blockIdx.x && blockIdx.x < a.more[min(i + per, a.n_bricks)]) group = i;
+        __syncthreads();
+        const uint32_t b = group + threadIdx.x;
+        if (threadIdx.x < per && b < a.n_bricks && a.more[b] <= blockIdx.x && blockIdx.x < a.more[b + 1u]) found = b;
+        __syncthreads();
+        brick = found;
+        part = blockIdx.x - a.more[brick] + 1u;
+    }
+    const uint32_t begin = a.start[brick] + part * kPartEntries, last = a.start[brick + 1u];
+    const uint32_t end = min(begin + kPartEntries, last);
+    const bool whole = part == 0u && end == last;
     for (uint32_t i = threadIdx.x; i < 512u; i += kBrickThreads) words[i][0] = words[i][1] = 0ull;
     __syncthreads();
 #pragma unroll 2
-    for (uint32_t e = first + threadIdx.x; e < end; e += kBrickThreads) {
+    for (uint32_t e = begin + threadIdx.x; e < end; e += kBrickThreads) {
         const unsigned long long w = a.entries[e];
         const long long x = (long long)((w >> 9) & 0x3ffffull) - 65536, y = (long long)((w >> 27) & 0x3ffffull) - 65536,
                         z = (long long)((w >> 45) & 0x3ffffull) - 65536;
@@ -193,15 +251,18 @@ vertex_brick_kernel(VertexBins a, uint32_t* __restrict__ counts, uint4* __restri
         atomicAdd(&words[w & 511u][1], (unsigned long long)(z) * (1ull << 32) + 1ull);
     }
     __syncthreads();
-    const uint32_t ox = 8u * (brick % a.bx), oy = 8u * (brick / a.bx % a.by), oz = 8u * (brick / (a.bx * a.by));
-    for (uint32_t i = threadIdx.x; i < 512u; i += kBrickThreads) {
-        const uint32_t x = ox + (i & 7u), y = oy + ((i >> 3) & 7u), z = oz + (i >> 6);
-        if (x >= a.g.nx || y >= a.g.ny || z >= a.g.nz) continue;
-        const size_t v = x + size_t(a.g.nx) * (y + size_t(a.g.ny) * z);
-        acc[v] = make_uint4(uint32_t(words[i][0]), uint32_t(words[i][0] >> 32), uint32_t(words[i][1]),
-                            uint32_t(words[i][1] >> 32));
-        if (counts) counts[v] = uint32_t(words[i][1]);
-    }
+    brick_voxels<kBrickThreads>(a, brick, [&](uint32_t i, size_t v) {
+        const unsigned long long w0 = words[i][0], w1 = words[i][1];
+        if (whole) {
+            a.acc[v] = make_uint4(uint32_t(w0), uint32_t(w0 >> 32), uint32_t(w1), uint32_t(w1 >> 32));
+            if (a.counts) a.counts[v] = uint32_t(w1);
+        } else if (uint32_t(w1) != 0u) {   // its count in this part
+            unsigned long long* sums = reinterpret_cast<unsigned long long*>(a.acc + v);
+            atomicAdd(&sums[0], w0);
+            atomicAdd(&sums[1], w1);
+            if (a.counts) atomicAdd(&a.counts[v], uint32_t(w1));
+        }
+    });
 }
 
 size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
@@ -222,7 +283,7 @@ int voxelize_vertices_binned(const float* xyz, uint32_t n_vertices, const float*
     a.blocks = (n_vertices + a.chunk - 1u) / a.chunk;
     const size_t hist = align256(size_t(a.blocks) * a.n_bricks * 4), total = align256(size_t(a.n_bricks) * 4),
                  start = align256((size_t(a.n_bricks) + 1) * 4);
-    const size_t bytes = hist + total + start + size_t(n_vertices) * 8;
+    const size_t bytes = hist + total + 2 * start + size_t(n_vertices) * 8;
     if (bytes > kBinScratch || capturing(s)) return VKHR_OK;
     const CallScratch temporaries(bytes, s);
     if (!temporaries.get()) return VKHR_OK;
@@ -234,7 +295,11 @@ int voxelize_vertices_binned(const float* xyz, uint32_t n_vertices, const float*
     a.hist = reinterpret_cast<uint32_t*>(p);
     a.total = reinterpret_cast<uint32_t*>(p + hist);
     a.start = reinterpret_cast<uint32_t*>(p + hist + total);
-    a.entries = reinterpret_cast<unsigned long long*>(p + hist + total + start);
+    a.more = reinterpret_cast<uint32_t*>(p + hist + total + start);
+    a.entries = reinterpret_cast<unsigned long long*>(p + hist + total + 2 * start);
+    a.more_blocks = n_vertices / kPartEntries;
+    a.counts = counts;
+    a.acc = reinterpret_cast<uint4*>(acc);
     const size_t lds = size_t(a.n_bricks) * 4;
     vertex_hist_kernel<<<a.blocks, kBinThreads, lds, s>>>(a);
     VKHR_CHECK_LAUNCH();
@@ -242,7 +307,7 @@ int voxelize_vertices_binned(const float* xyz, uint32_t n_vertices, const float*
     VKHR_CHECK_LAUNCH();
     vertex_fill_kernel<<<a.blocks, kBinThreads, lds, s>>>(a);
     VKHR_CHECK_LAUNCH();
-    vertex_brick_kernel<<<a.n_bricks, kBrickThreads, 0, s>>>(a, counts, reinterpret_cast<uint4*>(acc));
+    vertex_brick_kernel<<<a.more_blocks + a.n_bricks, kBrickThreads, 0, s>>>(a);
     VKHR_CHECK_LAUNCH();
     *taken = true;
     return VKHR_OK;
