@@ -73,25 +73,40 @@ aabb_final_kernel(const float* __restrict__ partial, int blocks, float* __restri
     }
 }
 
-// The two generators below give a strand to 16 lanes, which take its
-// vertices 16 at a time: a strand's vertices are consecutive, so a group
-// reads and writes whole lines, where a thread per strand spread every load
-// and store of a wave over 64 strands.  What bounds them is memory: at 136k
-// strands of 13 vertices (21 MB in, 21 MB out) the tangents take 13.9 us,
-// 51.4 with a thread per strand; the indices 7.5 us, 12.2 before.
-constexpr uint32_t kStrandLanes = 16;
+// The two generators below give a strand to a group of 1 to 16 lanes, the
+// power of two at or above the mean strand, which take its vertices (or pairs) that many
+// at a time: a strand's vertices are consecutive, so a group reads and writes
+// whole lines, where a thread per strand spread every load and store of a
+// wave over 64 strands.  What bounds them is memory: at 136k strands of 13
+// vertices (21 MB in, 21 MB out) the tangents take 13.9 us, 51.4 with a thread
+// per strand; the indices 7.5 us, 12.2 before.  Sixteen lanes whatever the
+// strands leave most of them idle on short ones: tangents of
+// 4M strands of two vertices 158 us (56 now), their indices 94 (27).
+constexpr uint32_t kMostLanes = 16, kStrandBlocks = 8192;
+
+// Calls strand(s, lane, lanes) for the strands of this lane's group; a strand
+// has its vertices less `less` items.
+template <typename Strand>
+__device__ __forceinline__ void each_strand(const uint32_t* __restrict__ offsets, uint32_t n_strands, uint32_t less,
+                                            Strand strand) {
+    const uint32_t mean = (offsets[n_strands] - offsets[0] - 1u) / n_strands + 1u - less;   // rounded up
+    const uint32_t shift = mean > 8u ? 4u : mean > 4u ? 3u : mean > 2u ? 2u : mean > 1u ? 1u : 0u, lanes = 1u << shift;
+    const uint32_t lane = threadIdx.x & (lanes - 1u), per_block = blockDim.x >> shift;
+    for (size_t s = size_t(blockIdx.x) * per_block + (threadIdx.x >> shift); s < n_strands;
+         s += size_t(gridDim.x) * per_block)
+        strand(uint32_t(s), lane, lanes);
+}
 
 __global__ void __launch_bounds__(256)
 indices_kernel(const uint32_t* __restrict__ offsets, uint32_t n_strands, uint32_t* __restrict__ indices) {
-    const uint32_t lane = threadIdx.x % kStrandLanes, per_block = blockDim.x / kStrandLanes;
-    for (uint32_t s = blockIdx.x * per_block + threadIdx.x / kStrandLanes; s < n_strands; s += gridDim.x * per_block) {
-        const uint32_t first = offsets[s], end = offsets[s + 1];
+    each_strand(offsets, n_strands, 1u, [&](uint32_t s, uint32_t lane, uint32_t lanes) {
+        const uint32_t first = offsets[s], end = offsets[s + 1u];
         const uint32_t out = 2u * (first - s);  // every earlier strand skipped its last vertex
-        for (uint32_t v = first + lane; v + 1u < end; v += kStrandLanes) {
+        for (uint32_t v = first + lane; v + 1u < end; v += lanes) {
             indices[out + 2u * (v - first)] = v;
             indices[out + 2u * (v - first) + 1u] = v + 1u;
         }
-    }
+    });
 }
 
 __device__ __forceinline__ float3 glm_normalize(float3 v) {
@@ -103,10 +118,9 @@ __device__ __forceinline__ float3 glm_normalize(float3 v) {
 __global__ void __launch_bounds__(256)
 tangents_kernel(const float* __restrict__ xyz, const uint32_t* __restrict__ offsets, uint32_t n_strands,
                 float* __restrict__ tangents) {
-    const uint32_t lane = threadIdx.x % kStrandLanes, per_block = blockDim.x / kStrandLanes;
-    for (uint32_t s = blockIdx.x * per_block + threadIdx.x / kStrandLanes; s < n_strands; s += gridDim.x * per_block) {
-        const uint32_t first = offsets[s], end = offsets[s + 1];
-        for (uint32_t v = first + lane; v < end; v += kStrandLanes) {
+    each_strand(offsets, n_strands, 0u, [&](uint32_t s, uint32_t lane, uint32_t lanes) {
+        const uint32_t first = offsets[s], end = offsets[s + 1u];
+        for (uint32_t v = first + lane; v < end; v += lanes) {
             // the strand's last vertex repeats the previous tangent
             const uint32_t a = v + 1u < end ? v : v - 1u;
             float3 t = make_float3(0.0f, 0.0f, 0.0f);
@@ -118,7 +132,7 @@ tangents_kernel(const float* __restrict__ xyz, const uint32_t* __restrict__ offs
             tangents[3u * v + 1u] = t.y;
             tangents[3u * v + 2u] = t.z;
         }
-    }
+    });
 }
 
 }  // namespace
@@ -170,8 +184,8 @@ extern "C" int vkhr_generate_indices(const uint32_t* strand_offsets, uint32_t n_
     if (rc) return rc;
     if (n_strands == 0) return VKHR_OK;
     VKHR_REQUIRE(strand_offsets && indices, VKHR_ERR_INVALID, "null pointer");
-    indices_kernel<<<grid_for(n_strands, 256 / kStrandLanes, 65536), 256, 0, as_stream(stream)>>>(strand_offsets, n_strands,
-                                                                                   indices);
+    indices_kernel<<<grid_for(n_strands, 256 / kMostLanes, kStrandBlocks), 256, 0, as_stream(stream)>>>(
+        strand_offsets, n_strands, indices);
     VKHR_CHECK_LAUNCH();
     return VKHR_OK;
 }
@@ -183,8 +197,8 @@ extern "C" int vkhr_generate_tangents(const float* xyz, const uint32_t* strand_o
     if (rc) return rc;
     if (n_strands == 0) return VKHR_OK;
     VKHR_REQUIRE(xyz && strand_offsets && tangents, VKHR_ERR_INVALID, "null pointer");
-    tangents_kernel<<<grid_for(n_strands, 256 / kStrandLanes, 65536), 256, 0, as_stream(stream)>>>(xyz, strand_offsets,
-                                                                                    n_strands, tangents);
+    tangents_kernel<<<grid_for(n_strands, 256 / kMostLanes, kStrandBlocks), 256, 0, as_stream(stream)>>>(
+        xyz, strand_offsets, n_strands, tangents);
     VKHR_CHECK_LAUNCH();
     return VKHR_OK;
 }
