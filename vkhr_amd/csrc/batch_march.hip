@@ -218,6 +218,7 @@ int build_group(vkhr_batch* b, const vkhr_batch_style* styles, uint32_t first, u
         vol.nx = vol.ny = vol.nz = in.volume;
         if ((rc = make_raymarch_args(&vol, &in.camera, &in.light, &in.strand, &in.params, width, height, &args[s])))
             return rc;
+        if (run_samples(args[s]) < kLeastRunSamples) args[s].n_segments = 0;   // (the power-of-two march reads none)
         args[s].rgba = reinterpret_cast<float4*>(in.rgba);
         lds_bytes = std::max(lds_bytes, distance_lds_bytes(args[s].vol));
         tile_prefix[s + 1] = tile_prefix[s] + tiles_x * tiles_y;

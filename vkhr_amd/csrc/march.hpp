@@ -765,6 +765,19 @@ __device__ double float_shadow_sum(const RaymarchArgs& a, const double xs[3], co
     return sum;
 }
 
+// Samples of a march over runs (0: not in that form).
+__host__ inline int run_samples(const RaymarchArgs& a) {
+    return a.n_segments ? a.segments[a.n_segments - 1].first + a.segments[a.n_segments - 1].count : 0;
+}
+
+// Step counts off the powers of two march over runs from this many samples on;
+// fewer take the shader's loop.  The runs are about two per doubling of the
+// parameter, and each needs a set-up that a dozen samples do not pay for
+// (1080p / 150^3, us, loop / runs: 24 steps 96 / 112, 48 115 / 131, 84 144 /
+// 152, 100 157 / 156; with four lanes per pixel, 160x90 / 250^3: 24 41 / 48,
+// 48 50.5 / 53, 56 53 / 53.5; 64^3: 56 50 / 45).
+constexpr int kLeastRunSamples = 96, kLeastQuadSamples = 56;
+
 // What the marches of one launch may take.
 enum MarchForm { kFormAny, kFormPower, kFormRuns };   // any; one run, or several (a.n_segments)
 

@@ -134,7 +134,8 @@ double smoothstep(double e0, double e1, double x) {
 static bool four_lanes_per_pixel(const RaymarchArgs& a) {
     const double pixels = double(a.width) * a.height, steps = std::fmin(1.0 / double(a.step_size), 512.0);
     if (a.vol.f32) return a.steps_per_unit > 0.0f && pixels <= 1400.0 * steps;
-    return !a.record && a.n_segments > 0 && pixels <= 800.0 * steps;
+    return !a.record && a.n_segments > 0 && (a.steps_per_unit > 0.0f || run_samples(a) >= kLeastQuadSamples) &&
+           pixels <= 800.0 * steps;
 }
 
 void launch_raymarch(const RaymarchArgs& a, hipStream_t stream) {
@@ -149,7 +150,7 @@ void launch_raymarch(const RaymarchArgs& a, hipStream_t stream) {
     }
     else if (four_lanes_per_pixel(a))
         raymarch_quad_kernel<<<dim3((a.width + 7) / 8, (a.height + 7) / 8), 256, lds, stream>>>(a);
-    else if (a.steps_per_unit > 0.0f)
+    else if (a.steps_per_unit > 0.0f || run_samples(a) < kLeastRunSamples)   // (or the shader's loop)
         raymarch_kernel<kFormPower><<<grid, 256, lds, stream>>>(a);
     else
         raymarch_kernel<kFormRuns><<<grid, 256, lds, stream>>>(a);
