@@ -62,7 +62,7 @@ struct RaymarchArgs {
     MarchRecord* record;
     PpllView ppll;             // node insertion when ppll.heads is set
     int n_segments;            // 0: the samples are not in that form
-    int reserved;
+    int run_part;              // samples of a run that share a fixed-point grid
     StepSegment segments[kMaxSegments];
 };
 
@@ -427,6 +427,27 @@ __device__ __forceinline__ uint32_t group_bits(bool v) {
     return uint32_t(m >> (__lane_id() & ~(kLanes - 1))) & ((1u << kLanes) - 1u);
 }
 
+// The parts of the runs, one after the other: at most a.run_part samples
+// each, since the grid of a part drifts from the float64 positions by 2^-33
+// texels a sample.  Calls part(segment) for each.
+template <typename Part>
+__device__ __forceinline__ void each_part(const RaymarchArgs& a, Part part) {
+    for (int s = 0, done = 0; s < a.n_segments;) {
+        StepSegment sg = a.segments[s];
+        sg.t0 = fma(double(done), sg.inc, sg.t0);
+        sg.first += done;
+        sg.count -= done;
+        if (sg.count > a.run_part) {
+            sg.count = a.run_part;
+            done += a.run_part;
+        } else {
+            ++s;
+            done = 0;
+        }
+        part(sg);
+    }
+}
+
 // A ray's grid on one run: sample j at texel coordinate + 1 p0 + j * d, and
 // the exits of empty brick regions in units of j.
 struct RunRay {
@@ -524,15 +545,14 @@ __device__ PrimaryMarch run_march(const RaymarchArgs& a, const Ray& ray, const O
 #pragma unroll
     for (int c = 0; c < 3; ++c) inv_dx[c] = 1.0 / ray.dx[c];
     bool settled = false, ended = false;  // settled: wave-uniform
-    for (int s = 0; s < a.n_segments; ++s) {
-        const StepSegment sg = a.segments[s];
+    each_part(a, [&](const StepSegment& sg) {
         int j, j_end;
         run_range(sg, t_lo, t_hi, &j, &j_end);
         const int j_depth = int(fmin(fmax(floor((t_depth - sg.t0) * sg.inv), 0.0), double(sg.count)));
         j = min(j, j_depth);
         if (j_depth < sg.count) j_end = sg.count;  // (the depth test also ends the count of samples)
-        if (ended || t_lo > t_hi && j_depth >= sg.count) j_end = 0;
-        if (j >= j_end) continue;
+        if (ended || (t_lo > t_hi && j_depth >= sg.count)) j_end = 0;
+        if (j >= j_end) return;
         const RunRay run = run_ray(sg, ray.xs, ray.dx, inv_dx, occ.use);
         long long P[3];
 #pragma unroll
@@ -601,7 +621,7 @@ __device__ PrimaryMarch run_march(const RaymarchArgs& a, const Ray& ray, const O
             j = next;
         }
         m.taken = sg.first + min(j, j_end);
-    }
+    });
     m.acc += group_sum<kLanes>(part);
     return m;
 }
@@ -615,11 +635,10 @@ __device__ double run_shadow_sum(const RaymarchArgs& a, const OccupancyView& occ
     double sum = 0.0, inv_dx[3];
 #pragma unroll
     for (int c = 0; c < 3; ++c) inv_dx[c] = 1.0 / dx[c];
-    for (int s = 0; s < a.n_segments; ++s) {
-        const StepSegment sg = a.segments[s];
+    each_part(a, [&](const StepSegment& sg) {
         int j, j_end;
         run_range(sg, t_lo, t_hi, &j, &j_end);
-        if (j >= j_end || t_lo > t_hi) continue;
+        if (j >= j_end || t_lo > t_hi) return;
         const RunRay run = run_ray(sg, xs, dx, inv_dx, occ.use);
         long long P[3];
 #pragma unroll
@@ -634,7 +653,7 @@ __device__ double run_shadow_sum(const RaymarchArgs& a, const OccupancyView& occ
             for (int c = 0; c < 3; ++c) P[c] += times(k, run.r.d[c]);
             j = next;
         }
-    }
+    });
     return group_sum<kLanes>(sum);
 }
 
