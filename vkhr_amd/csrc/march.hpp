@@ -561,10 +561,10 @@ __device__ PrimaryMarch run_march(const RaymarchArgs& a, const Ray& ray, const O
             float d[2];
             int next = 0;
             bool take = group_taps<kLanes>(vol, occ, run, P, q, j, j_end, d, &next);
-            if (!take && next > j_depth) {  // not past a sample of the depth test: its taps are 0
+            if (!take && next > j_depth) {  // not past a sample of the depth test: the region's taps are 0
                 take = true;
                 d[0] = d[1] = 0.0f;
-                next = j + 2 * kLanes;
+                next = min(next, j + 2 * kLanes);   // (what lies past the region is gathered next)
             }
             if (take) {
                 if (j + 2 * kLanes > j_depth) {
@@ -575,7 +575,8 @@ __device__ PrimaryMarch run_march(const RaymarchArgs& a, const Ray& ray, const O
                     for (int u = 0; u < 2; ++u) {
                         const int k = j + q + u * kLanes;
                         const double t = fma(double(k), sg.inc, sg.t0);
-                        behind[u] = k >= j_depth && k < j_end && db * fma(t, ray.dw, ray.ws) < fma(t, ray.dz, ray.zs);
+                        behind[u] = k >= j_depth && k < min(j_end, next) &&
+                                    db * fma(t, ray.dw, ray.ws) < fma(t, ray.dz, ray.zs);
                     }
                     const uint32_t mask = group_bits<kLanes>(behind[0]) | (group_bits<kLanes>(behind[1]) << kLanes);
                     if (mask != 0u) {
