@@ -67,7 +67,7 @@ segment_codes_kernel(const float* __restrict__ xyz, uint32_t n_vertices, const u
 // In every stage a block owns one contiguous chunk, in tiles of 4096 pairs or
 // 2048 runs, consecutive ones in each wave.
 constexpr int kOrderBlock = 1024, kOrderWaves = kOrderBlock / kWave, kOrderItems = 4;
-constexpr uint32_t kOrderTile = kOrderBlock * kOrderItems;   // pairs; runs when one tile holds them all
+constexpr uint32_t kOrderTile = kOrderBlock * kOrderItems;   // pairs
 // Runs per thread in a tile of the launches' passes.  Two keep enough
 // workgroups sorting: with 136k strands in tiles of 4096 there are 34, a
 // scatter taking 10.6 us against 8.0; eight were no faster at 12M runs.
@@ -78,10 +78,13 @@ constexpr int kDigits = 256, kPasses = 4;
 constexpr uint32_t kMaxRunBlocks = 2048, kMaxSortBlocks = 512;
 // Up to this many pairs one workgroup runs the stages over the runs in one
 // launch instead of ten: 17 us for 2k strands / 22k pairs, 52 in launches of
-// their own.  It holds kOrderTile runs; the host, which waits for the result
-// anyway, reads the run count with it and starts the launches when there
-// were more (32768 pairs of a run each: 120 us in all, 108 for the pairs' own sort before).
-constexpr uint32_t kOneBlockPairs = 32768;
+// their own.  It holds kTileRuns runs, in LDS; the host, which waits for the
+// result anyway, reads the run count with it and starts the launches when
+// there were more.  Workgroup against launches, pairs that are a run each (us
+// of the call): 4096 63 / 102, 5000 69 / 107, 10000 96 / 107, 15000 123 / 107.
+constexpr uint32_t kOneBlockPairs = 32768, kTileRuns = 10240;
+// Up to this many pairs that workgroup runs every stage (1000 pairs 43 -> 39 us)
+constexpr uint32_t kWholePairs = kOrderTile;
 
 struct OrderArgs {
     const float* xyz;
@@ -403,12 +406,12 @@ __device__ __forceinline__ void sum_lengths(const OrderArgs& a, OrderLds& lds, u
 // the lengths of the runs before each in the order.  Returns the lengths' sum.
 template <int kItems>
 __device__ __forceinline__ uint32_t tile_deltas(const OrderArgs& a, OrderLds& lds, const uint32_t (&run)[kItems],
-                                                uint32_t n, uint32_t base, uint32_t per = kItems) {
+                                                uint32_t n, uint32_t base) {
     const int lane = threadIdx.x % kWave;
     uint32_t first[kItems], len[kItems], at[kItems], wave_sum = 0;
 #pragma unroll
     for (int r = 0; r < kItems; ++r) {
-        const bool valid = uint32_t(r) < per && wave_item(0, r, per) < n;
+        const bool valid = wave_item(0, r, kItems) < n;
         first[r] = a.start[valid ? run[r] : 0u];
         len[r] = a.start[valid ? run[r] + 1u : 0u] - first[r];
         len[r] = valid ? len[r] : 0u;
@@ -427,7 +430,7 @@ __device__ __forceinline__ uint32_t tile_deltas(const OrderArgs& a, OrderLds& ld
     const uint32_t sum = block_sum(lds, lane == 0 ? wave_sum : 0u, &before);
 #pragma unroll
     for (int r = 0; r < kItems; ++r)
-        if (uint32_t(r) < per && wave_item(0, r, per) < n) a.delta[run[r]] = base + before + at[r] - first[r];
+        if (wave_item(0, r, kItems) < n) a.delta[run[r]] = base + before + at[r] - first[r];
     return sum;
 }
 
@@ -445,18 +448,19 @@ __device__ __forceinline__ void run_deltas(const OrderArgs& a, OrderLds& lds, ui
     }
 }
 
-// All passes over one tile's runs: they stay in registers, `per` to a lane,
-// and change places through LDS.
+// All passes over at most kTileRuns runs: they stay in registers, `per` to a
+// lane, and change places through LDS.
+constexpr int kTileItems = int(kTileRuns) / kOrderBlock;
 struct TileLds {
-    uint32_t key[kOrderTile], run[kOrderTile];
+    uint32_t key[kTileRuns], run[kTileRuns];
 };
 __device__ __forceinline__ void sort_tile(const OrderArgs& a, OrderLds& lds, TileLds& tile) {
     const uint32_t runs = *a.total, per = (runs + kOrderBlock - 1u) / kOrderBlock;
-    const int wave = threadIdx.x / kWave;
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
     const uint32_t digit = threadIdx.x % kDigits;
-    uint32_t key[kOrderItems], run[kOrderItems], rank[kOrderItems];
+    uint32_t key[kTileItems], run[kTileItems], rank[kTileItems];
 #pragma unroll
-    for (int r = 0; r < kOrderItems; ++r) {
+    for (int r = 0; r < kTileItems; ++r) {
         run[r] = wave_item(0, r, per);
         key[r] = uint32_t(r) < per && run[r] < runs ? a.keys[0][run[r]] : 0u;
     }
@@ -473,8 +477,9 @@ __device__ __forceinline__ void sort_tile(const OrderArgs& a, OrderLds& lds, Til
         if (threadIdx.x < kDigits) lds.base[digit] = first;
         __syncthreads();
 #pragma unroll
-        for (int r = 0; r < kOrderItems; ++r) {
-            if (uint32_t(r) >= per || wave_item(0, r, per) >= runs) continue;
+        for (int r = 0; r < kTileItems; ++r) {
+            if (uint32_t(r) >= per) break;
+            if (wave_item(0, r, per) >= runs) continue;
             const uint32_t d = (key[r] >> (8 * pass)) & (kDigits - 1u);
             const uint32_t at = lds.base[d] + lds.counts[wave][d] + rank[r];
             tile.key[at] = key[r];
@@ -482,13 +487,34 @@ __device__ __forceinline__ void sort_tile(const OrderArgs& a, OrderLds& lds, Til
         }
         __syncthreads();
 #pragma unroll
-        for (int r = 0; r < kOrderItems; ++r) {
-            if (uint32_t(r) >= per || wave_item(0, r, per) >= runs) continue;
+        for (int r = 0; r < kTileItems; ++r) {
+            if (uint32_t(r) >= per) break;
+            if (wave_item(0, r, per) >= runs) continue;
             key[r] = tile.key[wave_item(0, r, per)];
             run[r] = tile.run[wave_item(0, r, per)];
         }
     }
-    tile_deltas(a, lds, run, runs, 0u, per);
+    // where the runs' pairs go: the lengths of the runs before each in the order
+    uint32_t mine = 0;
+#pragma unroll
+    for (int r = 0; r < kTileItems; ++r) {
+        if (uint32_t(r) >= per) break;
+        rank[r] = wave_item(0, r, per) < runs ? run_length(a, run[r]) : 0u;
+        mine += rank[r];
+    }
+    uint32_t base;
+    block_sum(lds, mine, &base);
+#pragma unroll
+    for (int r = 0; r < kTileItems; ++r) {
+        if (uint32_t(r) >= per) break;
+        uint32_t scan = rank[r];
+        for (int o = 1; o < kWave; o <<= 1) {
+            const uint32_t below = __shfl_up(scan, o, kWave);
+            scan += lane >= o ? below : 0u;
+        }
+        if (wave_item(0, r, per) < runs) a.delta[run[r]] = base + scan - rank[r] - a.start[run[r]];
+        base += __shfl(scan, kWave - 1, kWave);
+    }
 }
 
 __device__ __forceinline__ void place_pairs(const OrderArgs& a, OrderLds& lds, uint32_t block) {
@@ -544,10 +570,21 @@ __global__ void __launch_bounds__(kOrderBlock) place_pairs_kernel(OrderArgs a, u
 __global__ void __launch_bounds__(kOrderBlock) order_tile_kernel(OrderArgs a) {
     __shared__ OrderLds lds;
     __shared__ TileLds tile;
-    if (*a.total <= kOrderTile) sort_tile(a, lds, tile);
+    if (*a.total <= kTileRuns) sort_tile(a, lds, tile);
 }
 
-// The same in launches of their own.
+// Every stage by one workgroup, which owns all pairs.
+__global__ void __launch_bounds__(kOrderBlock) order_whole_kernel(OrderArgs a) {
+    __shared__ OrderLds lds;
+    __shared__ TileLds tile;
+    emit_runs(a, lds, 0u);   // (the first block's runs need no count)
+    __syncthreads();
+    sort_tile(a, lds, tile);
+    __syncthreads();
+    place_pairs(a, lds, 0u);
+}
+
+// The stages over more runs in launches of their own.
 void launch_passes(const OrderArgs& a, hipStream_t s) {
     for (int pass = 0; pass < kPasses; ++pass) {
         count_digits_kernel<<<a.sort_blocks, kOrderBlock, 0, s>>>(a, pass);
@@ -647,8 +684,8 @@ extern "C" int vkhr_sort_strands(const float* xyz, uint32_t n_vertices, const ui
     a.n = n;
     a.box = *bounds;
     a.sorted = sorted;
-    const bool one = n <= kOneBlockPairs;
-    a.run_blocks = std::min((n + kOrderTile - 1u) / kOrderTile, kMaxRunBlocks);
+    const bool whole = n <= kWholePairs, one = n <= kOneBlockPairs;
+    a.run_blocks = whole ? 1u : std::min((n + kOrderTile - 1u) / kOrderTile, kMaxRunBlocks);
     a.run_chunk = ((n + a.run_blocks - 1u) / a.run_blocks + kOrderTile - 1u) / kOrderTile * kOrderTile;
     a.run_blocks = (n + a.run_chunk - 1u) / a.run_chunk;   // none empty
     a.sort_blocks = std::min((n + kSortTile - 1u) / kSortTile, kMaxSortBlocks);
@@ -676,13 +713,17 @@ extern "C" int vkhr_sort_strands(const float* xyz, uint32_t n_vertices, const ui
     a.delta = a.keys[0];
     HostWords host;
     a.host_total = host.words();
-    count_runs_kernel<<<a.run_blocks, kOrderBlock, 0, s>>>(a);
-    emit_runs_kernel<<<a.run_blocks, kOrderBlock, 0, s>>>(a);
     uint32_t runs = 0;
-    if (one) {
+    if (whole) {
+        order_whole_kernel<<<1, kOrderBlock, 0, s>>>(a);
+    } else {
+        count_runs_kernel<<<a.run_blocks, kOrderBlock, 0, s>>>(a);
+        emit_runs_kernel<<<a.run_blocks, kOrderBlock, 0, s>>>(a);
+    }
+    if (one && !whole) {
         order_tile_kernel<<<1, kOrderBlock, 0, s>>>(a);
-        place_pairs_kernel<<<a.run_blocks, kOrderBlock, 0, s>>>(a, kOrderTile);
-        if (n > kOrderTile) {
+        place_pairs_kernel<<<a.run_blocks, kOrderBlock, 0, s>>>(a, kTileRuns);
+        if (n > kTileRuns) {
             hipError_t c = hipSuccess;
             if (!host.words()) c = hipMemcpyAsync(&runs, a.total, sizeof(runs), hipMemcpyDeviceToHost, s);
             if (c == hipSuccess) c = hipStreamSynchronize(s);
@@ -690,7 +731,7 @@ extern "C" int vkhr_sort_strands(const float* xyz, uint32_t n_vertices, const ui
             VKHR_CHECK_HIP(c);
         }
     }
-    if (!one || runs > kOrderTile) {
+    if (!one || runs > kTileRuns) {
         launch_passes(a, s);
         place_pairs_kernel<<<a.run_blocks, kOrderBlock, 0, s>>>(a, n);
     }
