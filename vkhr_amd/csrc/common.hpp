@@ -79,6 +79,23 @@ int static_scratch(size_t bytes, void** out);
 // area is left, and the block of reuse_block.
 int release_stream_scratch(hipStream_t stream);
 
+// Allocations, frees and waits for a stream are refused on every thread, and
+// end the capture, while any thread captures in global mode, unless the thread
+// that makes them is in relaxed mode: they touch no captured stream.
+class RelaxedCapture {
+public:
+    RelaxedCapture() { ok_ = hipThreadExchangeStreamCaptureMode(&mode_) == hipSuccess; }
+    ~RelaxedCapture() {
+        if (ok_) (void)hipThreadExchangeStreamCaptureMode(&mode_);
+    }
+    RelaxedCapture(const RelaxedCapture&) = delete;
+    RelaxedCapture& operator=(const RelaxedCapture&) = delete;
+
+private:
+    hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;  // the thread's own once exchanged
+    bool ok_ = false;
+};
+
 // Temporaries that one call has to itself: the block that its stream keeps
 // for this, when it is there and large enough, else an allocation, which
 // becomes that block at the call's end if it is kKeptTemporaries or less and

@@ -677,6 +677,7 @@ extern "C" int vkhr_sort_strands(const float* xyz, uint32_t n_vertices, const ui
     hipStream_t s = as_stream(stream);
     VKHR_REQUIRE(!capturing(s), VKHR_ERR_HIP,
                  "strand sort failed: it synchronises the stream, which is being captured");
+    const RelaxedCapture relaxed;   // (it waits for the stream)
     OrderArgs a{};
     a.xyz = xyz;
     a.indices = indices;

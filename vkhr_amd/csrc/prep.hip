@@ -148,6 +148,7 @@ extern "C" int vkhr_aabb_compute(const float* xyz, uint32_t n_vertices, vkhr_aab
     VKHR_REQUIRE(n_vertices == 0 || xyz, VKHR_ERR_INVALID, "xyz is null");
     float mm[6] = {0, 0, 0, 0, 0, 0};
     if (n_vertices) {
+        const RelaxedCapture relaxed;   // (it waits for the stream)
         void* scr = nullptr;
         if ((rc = stream_scratch(sizeof(float) * (6 * kAabbGrid + 8), as_stream(stream), &scr))) return rc;
         float* partial = static_cast<float*>(scr);

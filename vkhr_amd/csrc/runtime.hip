@@ -51,23 +51,6 @@ Block g_kept[kMaxDevices];
 static __device__ __align__(256) uint32_t scratch[kStaticScratchBytes / sizeof(uint32_t)];
 void* g_static_scratch[kMaxDevices] = {nullptr};
 
-// Allocations and frees are refused on every thread, and end the capture,
-// while any thread captures in global mode, unless the thread that makes
-// them is in relaxed mode: they touch no captured stream.
-class RelaxedCapture {
-public:
-    RelaxedCapture() { ok_ = hipThreadExchangeStreamCaptureMode(&mode_) == hipSuccess; }
-    ~RelaxedCapture() {
-        if (ok_) (void)hipThreadExchangeStreamCaptureMode(&mode_);
-    }
-    RelaxedCapture(const RelaxedCapture&) = delete;
-    RelaxedCapture& operator=(const RelaxedCapture&) = delete;
-
-private:
-    hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;  // the thread's own once exchanged
-    bool ok_ = false;
-};
-
 ScratchKey scratch_key(int dev, hipStream_t stream) {
     const size_t thread = stream == hipStreamPerThread ? std::hash<std::thread::id>()(std::this_thread::get_id()) : 0;
     return ScratchKey(dev, stream, thread);
@@ -184,6 +167,7 @@ int release_stream_scratch(hipStream_t stream) {
         }
         if (g_scratch.empty() && g_host_used == 0) std::swap(page, g_host_page);
     }
+    const RelaxedCapture relaxed;
     if (page) VKHR_CHECK_HIP(hipHostFree(page));
     if (block.ptr) VKHR_CHECK_HIP(hipFree(block.ptr));
     if (!found) return VKHR_OK;
@@ -235,10 +219,11 @@ void* reuse_block(int device, size_t bytes, size_t* held) {
     }
     // Frees wait for the device as hipDeviceSynchronize does, but unlike it
     // they leave a capture that another thread has under way valid.
+    const RelaxedCapture relaxed;
     void* token = nullptr;
     if (hipMalloc(&token, 256) != hipSuccess || hipFree(token) != hipSuccess) {
         (void)hipGetLastError();
-        (void)hipFree(block.ptr);
+        if (!keep_block(device, block.ptr, block.bytes)) (void)hipFree(block.ptr);
         return nullptr;
     }
     *held = block.bytes;

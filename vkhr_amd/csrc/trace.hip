@@ -1015,6 +1015,7 @@ extern "C" int vkhr_bvh_build(const float* xyz, const float* radius, uint32_t n_
                         2 * carve_size(inner * sizeof(uint32_t)) + carve_size(8 * inner * sizeof(uint32_t)) +
                         carve_size(sort_bytes);
     hipError_t e = hipSuccess;
+    const RelaxedCapture relaxed;
     b->memory = reuse_block(device, keep, &b->bytes);
     if (!b->memory) {
         b->bytes = keep;
@@ -1104,6 +1105,7 @@ extern "C" int vkhr_bvh_destroy(vkhr_bvh* b) {
     int prev = 0;
     (void)hipGetDevice(&prev);
     (void)hipSetDevice(b->device);
+    const RelaxedCapture relaxed;
     if (b->memory && !keep_block(b->device, b->memory, b->bytes)) (void)hipFree(b->memory);
     (void)hipSetDevice(prev);
     delete b;
