@@ -143,8 +143,9 @@ private:
 };
 
 // Device memory of an object that is often destroyed and built again (a
-// style's tree each frame): keep_block takes over a block to be freed, one
-// per device and at most kKeptTemporaries bytes (false: free it yourself),
+// style's tree each frame): keep_block takes over a block to be freed, of at
+// most kKeptTemporaries bytes (false: free it yourself), in place of the
+// device's last one, which it frees,
 // and reuse_block hands it out again when it holds `bytes` and is at most
 // four times that, once the device has finished everything that was queued
 // while the block was in use.  With the temporaries kept as well and the

@@ -203,9 +203,15 @@ HostWords::~HostWords() {
 
 bool keep_block(int device, void* ptr, size_t bytes) {
     if (device < 0 || device >= kMaxDevices || bytes > kKeptTemporaries) return false;
-    std::lock_guard<std::mutex> lock(g_mutex);
-    if (g_kept[device].ptr) return false;
-    g_kept[device] = Block{ptr, bytes};
+    Block block{ptr, bytes};
+    {
+        std::lock_guard<std::mutex> lock(g_mutex);
+        std::swap(block, g_kept[device]);
+    }
+    if (block.ptr) {
+        const RelaxedCapture relaxed;
+        (void)hipFree(block.ptr);
+    }
     return true;
 }
 
