@@ -317,8 +317,9 @@ constexpr int kFoldRows = 2, kFoldLevels = 8;
 __global__ void __launch_bounds__(256)
 gather_cells_kernel(const float* __restrict__ cg, const float* __restrict__ texels, float* __restrict__ grad, int nx,
                     int ny, int nz, const double* __restrict__ param_sums, float* __restrict__ d_params) {
+    // (atomic: calls on other streams may add to the same parameters)
     if (blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x < 3)
-        d_params[threadIdx.x] += float(param_sums[threadIdx.x]);
+        atomicAdd(&d_params[threadIdx.x], float(param_sums[threadIdx.x]));
     const int lane = threadIdx.x % kWave;
     const int x = int(blockIdx.x) * kWave + lane;
     const int y0 = (int(blockIdx.y) * (256 / kWave) + int(threadIdx.x) / kWave) * kFoldRows;
