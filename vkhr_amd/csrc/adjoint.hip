@@ -554,14 +554,15 @@ adjoint_cells_kernel(AdjointArgs) {
 
 struct AdjointBatchStyle {
     float* cell_grad;           // 8 floats per cell, owned by the batch
+    float* texel_grad;          // what the windows are flushed to, in the cells' pitch, behind them (nullable)
     float* d_density;
     float* d_params;
     uint32_t nx, ny, nz;
     uint32_t reserved;
 };
 
-// A contiguous range [begin, end) of one style's cell-accumulator floats
-// (clear) or voxels (fold).
+// A contiguous range [begin, end) of one style's accumulator floats, cells and
+// texels (clear), or voxels (fold).
 struct AdjointChunk {
     uint32_t style;
     uint32_t reserved;
@@ -591,12 +592,6 @@ adjoint_batch_clear_kernel(AdjointBatchDevice d) {
         const AdjointChunk ch = d.clear_chunks[c];
         float* cg = d.styles[ch.style].cell_grad;
         for (uint64_t i = ch.begin + threadIdx.x; i < ch.end; i += blockDim.x) cg[i] = 0.0f;
-    }
-    // the windows of the primary rays are flushed to d_density itself
-    for (uint32_t c = blockIdx.x; c < d.n_fold_chunks; c += gridDim.x) {
-        const AdjointChunk ch = d.fold_chunks[c];
-        float* g = d.styles[ch.style].d_density;
-        for (uint64_t i = ch.begin + threadIdx.x; i < ch.end; i += blockDim.x) g[i] = 0.0f;
     }
 }
 
@@ -637,7 +632,7 @@ adjoint_batch_cells_kernel(AdjointBatchDevice d, const AdjointArgs* __restrict__
     adjoint_batch_block<CellLds>(d, args, d.n_windows);
 }
 
-// d_density += the fold of each style's cells.
+// d_density = the fold of each style's cells and texels (overwritten).
 __global__ void __launch_bounds__(256)
 adjoint_batch_fold_kernel(AdjointBatchDevice d) {
     for (uint32_t c = blockIdx.x; c < d.n_fold_chunks; c += gridDim.x) {
@@ -646,7 +641,7 @@ adjoint_batch_fold_kernel(AdjointBatchDevice d) {
         const size_t cx = size_t(st.nx) + 1, cy = size_t(st.ny) + 1;
         for (uint64_t i = ch.begin + threadIdx.x; i < ch.end; i += blockDim.x) {
             const size_t x = i % st.nx, yz = i / st.nx, y = yz % st.ny, z = yz / st.ny;
-            float sum = st.d_density[i];
+            float sum = st.texel_grad ? st.texel_grad[x + cx * (y + cy * z)] : 0.0f;
 #pragma unroll
             for (int q = 0; q < 8; ++q) {
                 const size_t cell = (x + 1 - (q & 1)) + cx * ((y + 1 - ((q >> 1) & 1)) + cy * (z + 1 - (q >> 2)));
@@ -824,6 +819,8 @@ int build_adjoint_batch(vkhr_adjoint_batch* b, const vkhr_adjoint_style* styles,
     int rc = VKHR_OK;
     std::vector<AdjointBatchStyle> st(n_styles);
     std::vector<AdjointChunk> clear, fold;
+    std::vector<uint64_t> n_cells(n_styles);
+    std::vector<bool> windows(n_styles, false);   // some render of the style takes them
     const uint64_t kChunk = 1u << 16;
     for (uint32_t s = 0; s < n_styles; ++s) {
         const vkhr_adjoint_style& in = styles[s];
@@ -831,11 +828,8 @@ int build_adjoint_batch(vkhr_adjoint_batch* b, const vkhr_adjoint_style* styles,
                      "style %u: the float density, tangents, d_density and d_params are required", s);
         if ((rc = check_volume(in.volume.nx, in.volume.ny, in.volume.nz, true, "adjoint style volume"))) return rc;
         const uint64_t cells = (uint64_t(in.volume.nx) + 1) * (uint64_t(in.volume.ny) + 1) * (uint64_t(in.volume.nz) + 1);
-        void* cg = nullptr;
-        VKHR_CHECK_HIP(hipMalloc(&cg, cells * 8 * sizeof(float)));
-        b->allocations.push_back(cg);
-        st[s] = {static_cast<float*>(cg), in.d_density, in.d_params, in.volume.nx, in.volume.ny, in.volume.nz, 0};
-        for (uint64_t a = 0; a < cells * 8; a += kChunk) clear.push_back({s, 0, a, std::min(cells * 8, a + kChunk)});
+        n_cells[s] = cells;
+        st[s] = {nullptr, nullptr, in.d_density, in.d_params, in.volume.nx, in.volume.ny, in.volume.nz, 0};
         const uint64_t vox = uint64_t(in.volume.nx) * in.volume.ny * in.volume.nz;
         for (uint64_t a = 0; a < vox; a += kChunk) fold.push_back({s, 0, a, std::min(vox, a + kChunk)});
     }
@@ -857,13 +851,28 @@ int build_adjoint_batch(vkhr_adjoint_batch* b, const vkhr_adjoint_style* styles,
         a.target = reinterpret_cast<const float4*>(in.target);
         a.loss = in.loss;
         a.d_params = styles[in.style].d_params;
-        a.cell_grad = st[in.style].cell_grad;
-        a.texel_grad = st[in.style].d_density;
-        a.texel_row = size_t(a.f.nx);
-        a.texel_slice = size_t(a.f.nx) * a.f.ny;
+        a.texel_row = size_t(a.f.nx) + 1;
+        a.texel_slice = a.texel_row * (size_t(a.f.ny) + 1);
         finish_adjoint_args(&a);
         losses[r] = in.loss;
-        (window_scatter(a.f, in.camera) ? order : in_cells).push_back(r);
+        const bool in_windows = window_scatter(a.f, in.camera);
+        if (in_windows) windows[in.style] = true;
+        (in_windows ? order : in_cells).push_back(r);
+    }
+    // the accumulators: atomics go to memory of the batch's own (float atomics
+    // to a caller's fine-grained memory would be lost)
+    for (uint32_t s = 0; s < n_styles; ++s) {
+        const uint64_t floats = n_cells[s] * (windows[s] ? 9 : 8);
+        void* cg = nullptr;
+        VKHR_CHECK_HIP(hipMalloc(&cg, floats * sizeof(float)));
+        b->allocations.push_back(cg);
+        st[s].cell_grad = static_cast<float*>(cg);
+        if (windows[s]) st[s].texel_grad = st[s].cell_grad + n_cells[s] * 8;
+        for (uint64_t a = 0; a < floats; a += kChunk) clear.push_back({s, 0, a, std::min(floats, a + kChunk)});
+    }
+    for (uint32_t r = 0; r < n_renders; ++r) {
+        args[r].cell_grad = st[renders[r].style].cell_grad;
+        args[r].texel_grad = st[renders[r].style].texel_grad;
     }
     const uint32_t n_windows = uint32_t(order.size());
     order.insert(order.end(), in_cells.begin(), in_cells.end());
