@@ -962,6 +962,11 @@ T* carve(char*& p, size_t count) {
 
 size_t carve_size(size_t bytes) { return (bytes + 255) & ~size_t(255); }
 
+// The build's kernels take an element per thread, without a stride: their
+// launches hold every element of the largest tree (at most 2^22 workgroups).
+constexpr uint32_t kMostSegments = (1u << 30) - 1u;   // int range search in the tree build
+unsigned blocks_of(size_t n, unsigned block) { return unsigned((n + block - 1) / block); }
+
 }  // namespace
 
 extern "C" int vkhr_bvh_build(const float* xyz, const float* radius, uint32_t n_vertices, const uint32_t* indices,
@@ -976,7 +981,7 @@ extern "C" int vkhr_bvh_build(const float* xyz, const float* radius, uint32_t n_
     const auto plausible = [](const void* p) { return reinterpret_cast<uintptr_t>(p) >= 65536u; };
     VKHR_REQUIRE(n == 0 || (plausible(xyz) && plausible(radius) && plausible(indices)), VKHR_ERR_INVALID,
                  "null or implausible geometry pointer");
-    VKHR_REQUIRE(n < (1u << 30), VKHR_ERR_OVERFLOW, "too many segments");  // int range search in the tree build
+    VKHR_REQUIRE(n <= kMostSegments, VKHR_ERR_OVERFLOW, "too many segments");
     hipStream_t s = as_stream(stream);
     VKHR_REQUIRE(n == 0 || !capturing(s), VKHR_ERR_HIP,
                  "bvh build synchronises its stream, which is being captured");
@@ -992,7 +997,7 @@ extern "C" int vkhr_bvh_build(const float* xyz, const float* radius, uint32_t n_
     const size_t inner = n > 1 ? n - 1 : 0;
     const size_t keep = carve_size((inner + n) * sizeof(WideNode)) + carve_size(inner * 4 * sizeof(float4)) +
                         carve_size((inner + n) * sizeof(uint32_t)) + carve_size(n * sizeof(uint32_t));
-    const uint32_t blocks = grid_for(n, 256);
+    const uint32_t blocks = blocks_of(n, 256);
     // temporaries: boxes (input order), the pyramid of leaf boxes, bounds, keys/values x2, sort scratch
     size_t sort_bytes = 0;
     if (rocprim::radix_sort_pairs(nullptr, sort_bytes, static_cast<uint32_t*>(nullptr),
@@ -1074,14 +1079,14 @@ extern "C" int vkhr_bvh_build(const float* xyz, const float* radius, uint32_t n_
         set_error("bvh sort failed");
         return fail(VKHR_ERR_HIP);
     }
-    leaves_kernel<<<grid_for(n, kPyramidBlock, 1u << 21), kPyramidBlock, 0, s>>>(a, order, pyr, prims, b->prim_seg, made);
+    leaves_kernel<<<blocks_of(n, kPyramidBlock), kPyramidBlock, 0, s>>>(a, order, pyr, prims, b->prim_seg, made);
     if (n > 1) {
         for (int in = 3; in + 1 < pyr.levels; in += 3)
-            pyramid_kernel<<<grid_for(size_t(pyr.count[in]), kPyramidBlock), kPyramidBlock, 0, s>>>(pyr, in);
-        radix_tree_kernel<<<grid_for(inner, 256, 1u << 22), 256, 0, s>>>(keys_sorted, int(n), pyr, b->nodes, b->parent, ranges);
+            pyramid_kernel<<<blocks_of(size_t(pyr.count[in]), kPyramidBlock), kPyramidBlock, 0, s>>>(pyr, in);
+        radix_tree_kernel<<<blocks_of(inner, 256), 256, 0, s>>>(keys_sorted, int(n), pyr, b->nodes, b->parent, ranges);
         const WideArgs wa{keys_sorted, b->nodes, b->parent, ranges, int(n), a.bounds, prims, b->prim_seg,
                           made, place, base, sides, b->units};
-        const uint32_t wide_blocks = grid_for(inner, kWideBlock);
+        const uint32_t wide_blocks = blocks_of(inner, kWideBlock);
         wide_place_kernel<<<wide_blocks, kWideBlock, 0, s>>>(wa);
         wide_nodes_kernel<<<wide_blocks, kWideBlock, 0, s>>>(wa);
     } else {
