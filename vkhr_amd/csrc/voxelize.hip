@@ -78,6 +78,12 @@ constexpr uint32_t kPartEntries = 4096;
 constexpr uint32_t kBinVertices = 250000;
 constexpr size_t kBinScratch = kKeptTemporaries;
 
+// Vertices of a block: whole rounds of its threads, at most kBinBlocks blocks.
+constexpr uint32_t bin_chunk(uint32_t n_vertices) {
+    return uint32_t((uint64_t(n_vertices) + kBinBlocks * kBinThreads - 1u) / (kBinBlocks * kBinThreads)) * kBinThreads;
+}
+static_assert(bin_chunk(1) == kBinThreads && bin_chunk(0xffffffffu) >= 0xffffffffu / kBinBlocks, "no wrap, no zero");
+
 struct VertexBins {
     VoxelGrid g;
     const float* xyz;
@@ -279,8 +285,8 @@ int voxelize_vertices_binned(const float* xyz, uint32_t n_vertices, const float*
     a.n_bricks = a.bx * a.by * ((g.nz + 7u) >> 3);
     if (n_vertices < kBinVertices || a.n_bricks > kBinBricks || reinterpret_cast<uintptr_t>(acc) % 16 != 0)
         return VKHR_OK;
-    a.chunk = ((n_vertices + kBinBlocks - 1u) / kBinBlocks + kBinThreads - 1u) / kBinThreads * kBinThreads;
-    a.blocks = (n_vertices + a.chunk - 1u) / a.chunk;
+    a.chunk = bin_chunk(n_vertices);
+    a.blocks = (n_vertices - 1u) / a.chunk + 1u;
     const size_t hist = align256(size_t(a.blocks) * a.n_bricks * 4), total = align256(size_t(a.n_bricks) * 4),
                  start = align256((size_t(a.n_bricks) + 1) * 4);
     const size_t bytes = hist + total + 2 * start + size_t(n_vertices) * 8;
