@@ -18,7 +18,7 @@ struct MarchRecord {
     float shade[3];        // shading (Kajiya-Kay or 1)
     float spec_base;       // Kajiya-Kay specular base max(cTL cTE + sTL sTE, 0)
     int n_primary;         // samples taken by the primary march (up to the depth-buffer break or
-                           // the end of the volume's support)
+                           // the end of the volume's support, or a few samples past that end)
     int state;             // 0 miss, 1 fragment, 2 marched and discarded
 };
 static_assert(sizeof(MarchRecord) == 64, "record layout");

@@ -126,8 +126,10 @@ double smoothstep(double e0, double e1, double x) {
 // steps: 320x240 139 / 74, 640x360 137 / 104, 800x450 162 / 134, 960x540
 // 163 / 169, 1920x1080 283 / 544; 64^3, 128 steps: 320x240 43 / 38, 480x270
 // 44 / 51: the line falls with the march's share of the work, the step
-// count.  A record needs the count of samples as the loop takes them, which
-// the marches over runs do not keep.  A sample of the float volume takes
+// count.  It holds for counts of several runs too (150^3, 300 steps: 480x270
+// 138 / 102, 560x420 142 / 130, 640x480 141 / 152; 100 steps: 320x240 75 / 65,
+// 400x300 76 / 79).  A record of the cells takes one lane: none was measured
+// with four.  A sample of the float volume takes
 // about twice the work (128^3, 256 steps: 256^2 169 / 76, 512^2 195 / 174,
 // 640^2 232 / 241; 64^3, 128 steps: 384^2 86 / 73, 512^2 98 / 114); its
 // marches of other step counts take one lane.
