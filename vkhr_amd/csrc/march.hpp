@@ -31,7 +31,15 @@ struct StepSegment {
     double t0, inc, inv;       // inv = 1 / inc
     int first, count;
 };
-constexpr int kMaxSegments = 40;   // at most two per binade of t from 2^-17 up
+// A fixed-point grid drifts from the float64 positions by 2^-33 texels a
+// sample, so runs are cut at kRunPart samples: within 3e-8 texels, a float32
+// weight's rounding (at 65,000 steps over 250^3 the image is 8e-8 from float64
+// that way, 7.5e-6 with a grid per run).  A power-of-two count is one run
+// whatever its length, in every form, so that its images agree.
+constexpr int kRunPart = 256;
+// Two runs per binade of t from 2^-17 up at most, and the cuts of 11,000 steps;
+// counts that need more take the shader's loop.
+constexpr int kMaxSegments = 80;
 
 struct RaymarchArgs {
     double ivp[16];            // inverse(projection * view), column-major
@@ -62,7 +70,7 @@ struct RaymarchArgs {
     MarchRecord* record;
     PpllView ppll;             // node insertion when ppll.heads is set
     int n_segments;            // 0: the samples are not in that form
-    int run_part;              // samples of a run that share a fixed-point grid
+    int reserved;
     StepSegment segments[kMaxSegments];
 };
 
@@ -427,27 +435,6 @@ __device__ __forceinline__ uint32_t group_bits(bool v) {
     return uint32_t(m >> (__lane_id() & ~(kLanes - 1))) & ((1u << kLanes) - 1u);
 }
 
-// The parts of the runs, one after the other: at most a.run_part samples
-// each, since the grid of a part drifts from the float64 positions by 2^-33
-// texels a sample.  Calls part(segment) for each.
-template <typename Part>
-__device__ __forceinline__ void each_part(const RaymarchArgs& a, Part part) {
-    for (int s = 0, done = 0; s < a.n_segments;) {
-        StepSegment sg = a.segments[s];
-        sg.t0 = fma(double(done), sg.inc, sg.t0);
-        sg.first += done;
-        sg.count -= done;
-        if (sg.count > a.run_part) {
-            sg.count = a.run_part;
-            done += a.run_part;
-        } else {
-            ++s;
-            done = 0;
-        }
-        part(sg);
-    }
-}
-
 // A ray's grid on one run: sample j at texel coordinate + 1 p0 + j * d, and
 // the exits of empty brick regions in units of j.
 struct RunRay {
@@ -545,14 +532,15 @@ __device__ PrimaryMarch run_march(const RaymarchArgs& a, const Ray& ray, const O
 #pragma unroll
     for (int c = 0; c < 3; ++c) inv_dx[c] = 1.0 / ray.dx[c];
     bool settled = false, ended = false;  // settled: wave-uniform
-    each_part(a, [&](const StepSegment& sg) {
+    for (int s = 0; s < a.n_segments; ++s) {
+        const StepSegment sg = a.segments[s];
         int j, j_end;
         run_range(sg, t_lo, t_hi, &j, &j_end);
         const int j_depth = int(fmin(fmax(floor((t_depth - sg.t0) * sg.inv), 0.0), double(sg.count)));
         j = min(j, j_depth);
         if (j_depth < sg.count) j_end = sg.count;  // (the depth test also ends the count of samples)
         if (ended || (t_lo > t_hi && j_depth >= sg.count)) j_end = 0;
-        if (j >= j_end) return;
+        if (j >= j_end) continue;
         const RunRay run = run_ray(sg, ray.xs, ray.dx, inv_dx, occ.use);
         long long P[3];
 #pragma unroll
@@ -622,7 +610,7 @@ __device__ PrimaryMarch run_march(const RaymarchArgs& a, const Ray& ray, const O
             j = next;
         }
         m.taken = sg.first + min(j, j_end);
-    });
+    }
     m.acc += group_sum<kLanes>(part);
     return m;
 }
@@ -636,10 +624,11 @@ __device__ double run_shadow_sum(const RaymarchArgs& a, const OccupancyView& occ
     double sum = 0.0, inv_dx[3];
 #pragma unroll
     for (int c = 0; c < 3; ++c) inv_dx[c] = 1.0 / dx[c];
-    each_part(a, [&](const StepSegment& sg) {
+    for (int s = 0; s < a.n_segments; ++s) {
+        const StepSegment sg = a.segments[s];
         int j, j_end;
         run_range(sg, t_lo, t_hi, &j, &j_end);
-        if (j >= j_end || t_lo > t_hi) return;
+        if (j >= j_end || t_lo > t_hi) continue;
         const RunRay run = run_ray(sg, xs, dx, inv_dx, occ.use);
         long long P[3];
 #pragma unroll
@@ -654,7 +643,7 @@ __device__ double run_shadow_sum(const RaymarchArgs& a, const OccupancyView& occ
             for (int c = 0; c < 3; ++c) P[c] += times(k, run.r.d[c]);
             j = next;
         }
-    });
+    }
     return group_sum<kLanes>(sum);
 }
 

@@ -217,12 +217,16 @@ int make_raymarch_args(const vkhr_volume* vol, const vkhr_camera* cam, const vkh
         a->steps_per_unit = (m == 0.5f && s >= 1.0f && s <= 1048576.0f) ? s : 0.0f;
     }
     {
-        // the samples of the shader's loop as runs of equal increments
+        // the samples of the shader's loop as runs of equal increments, cut at
+        // kRunPart samples
         StepSegment* sg = nullptr;
         int n = 0, i = 0;
         for (float t = 0.0f; t < 1.0f; ++i) {
-            if (!sg || double(t) != sg->t0 + sg->count * sg->inc) {
-                if (n == kMaxSegments) break;
+            if (!sg || sg->count == kRunPart || double(t) != sg->t0 + sg->count * sg->inc) {
+                if (n == kMaxSegments) {
+                    n = 0;   // not in the form: the march takes the loop itself
+                    break;
+                }
                 sg = &a->segments[n++];
                 sg->t0 = t;
                 sg->inc = double(t + a->step_size) - double(t);
@@ -236,18 +240,13 @@ int make_raymarch_args(const vkhr_volume* vol, const vkhr_camera* cam, const vkh
             }
             ++sg->count;
             const float next = t + a->step_size;
-            if (next == t || (n == kMaxSegments && double(next) != sg->t0 + sg->count * sg->inc && next < 1.0f)) {
-                n = 0;   // not in the form: the march takes the loop itself
+            if (next == t) {
+                n = 0;
                 break;
             }
             t = next;
         }
         a->n_segments = n;
-        // Parts of 256 samples keep the positions within 3e-8 texels, a float32
-        // weight's rounding, at any count: at 65,000 steps over 250^3 the image
-        // is 8e-8 from float64, 7.5e-6 with a run's one grid.  (A power-of-two count
-        // is one grid in every form, so that its images agree.)
-        a->run_part = a->steps_per_unit > 0.0f ? 1 << 30 : 256;
     }
     a->shading_model = rp->shading_model;
     a->adsm_on = rp->adsm_on;
