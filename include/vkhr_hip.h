@@ -147,8 +147,7 @@ int vkhr_init(void);
  * counterpart in the reference (which keeps no device scratch). */
 int vkhr_release_scratch(vkhr_stream stream);
 /* Bytes of the scratch area held for this stream on the current device, with
- * the temporaries kept for it (0
- * when none). */
+ * the temporaries kept for it (0 when none). */
 size_t vkhr_scratch_bytes(vkhr_stream stream);
 
 /* ------------------------------------------------------ style preparation */
@@ -278,9 +277,9 @@ int vkhr_voxelize_segments(const float* xyz, uint32_t n_vertices,
  *                  distance - 1 is empty; all 0 when a side exceeds 2040, and
  *                  then nothing is skipped); then ceil(B/4) words the finalize
  *                  works in.  The raymarcher skips the gathers of samples in
- *                  empty bricks and, on the power-of-two sample grid, jumps
- *                  over empty brick regions (their taps read 0: the result is
- *                  unchanged). */
+ *                  empty bricks and, where it marches a grid of samples (a
+ *                  power-of-two count, or 96 and more), jumps over empty brick
+ *                  regions (their taps read 0: the result is unchanged). */
 int vkhr_volume_finalize(const uint32_t* counts, const int64_t* tangent_acc,
                          uint32_t nx, uint32_t ny, uint32_t nz, int normalize,
                          uint8_t* density_u8, int8_t* tangent_i8x4,
@@ -425,7 +424,8 @@ int vkhr_raymarch_record(const vkhr_volume* volume, const vkhr_camera* camera, c
  * choices are piecewise constant (no gradient); clamps pass gradient strictly
  * inside [0,1].  Rays are re-walked in short chunks from the ray set-up;
  * nothing per sample is stored.  Float atomics: summation order is not
- * deterministic. */
+ * deterministic.  d_params is added to atomically (calls on several streams
+ * may share it, in device memory); d_density is not. */
 int vkhr_raymarch_adjoint(const vkhr_volume* volume, const vkhr_camera* camera, const vkhr_light* light,
                           const vkhr_strand_params* strand, const vkhr_render_params* params,
                           const vkhr_diff_params* diff, uint32_t width, uint32_t height, const void* record,
@@ -619,8 +619,10 @@ typedef struct vkhr_adjoint_render {
 
 typedef struct vkhr_adjoint_batch vkhr_adjoint_batch;
 
-/* Builds the device tables and the per-style cell accumulators (8 floats
- * per cell of each style, owned by the batch). */
+/* Builds the device tables and the per-style accumulators (8 floats per cell
+ * of each style, 9 when some render's primary samples go through windows of
+ * texels; owned by the batch, which alone sees float atomics: d_density may
+ * be any memory the device writes). */
 int vkhr_adjoint_batch_create(const vkhr_adjoint_style* styles, uint32_t n_styles,
                               const vkhr_adjoint_render* renders, uint32_t n_renders, uint32_t width,
                               uint32_t height, vkhr_adjoint_batch** out);
@@ -628,7 +630,7 @@ int vkhr_adjoint_batch_create(const vkhr_adjoint_style* styles, uint32_t n_style
 /* Runs the step as one hipGraph (captured on the first call on a created,
  * non-NULL stream): clear, forward of all renders, adjoint of all renders
  * (the loss gradient 2 (rgba - target) is formed in the adjoint), and the
- * fold of each style's cells into its d_density.  The images and records
+ * fold of each style's accumulators into its d_density.  The images and records
  * are bit-identical to per-render vkhr_raymarch_record; the gradients equal
  * the sums of per-render vkhr_raymarch_adjoint up to float summation order. */
 int vkhr_adjoint_batch_launch(vkhr_adjoint_batch* batch, vkhr_stream stream);
@@ -673,8 +675,10 @@ typedef struct vkhr_trace_params {
 typedef struct vkhr_bvh vkhr_bvh;
 
 /* Builds the BVH of the segments of one style on the device (a linear BVH:
- * Morton-sorted leaves, binary radix tree, bottom-up boxes); the positions
- * and radii are copied into it, so the inputs may change afterwards.
+ * Morton-sorted leaves, binary radix tree, the eight-child nodes that rays
+ * visit cut from it; 204 bytes a segment); the positions and radii are
+ * copied into it, so the inputs may change afterwards.  Fewer than 2^30
+ * segments.
  * Synchronises the stream (load-time call); allocates, or takes over the
  * memory of the last tree destroyed once the device has gone idle. */
 int vkhr_bvh_build(const float* xyz, const float* radius, uint32_t n_vertices, const uint32_t* indices,

@@ -327,14 +327,6 @@ __device__ __forceinline__ float fixed_cells_blend(unsigned long long q, uint32_
     return cell_value(q, float(fx) * kInv, float(fy) * kInv, float(fz) * kInv);
 }
 
-// One trilinear tap of the cells at cell (cx, cy, cz) (texel + 1, inside
-// the support) with fractions (fx, fy, fz) in units of 2^-32.
-__device__ __forceinline__ float fixed_cells_tap(const DensityVolume& v, uint32_t cx, uint32_t cy, uint32_t cz,
-                                                 uint32_t fx, uint32_t fy, uint32_t fz) {
-    const uint32_t c = index24(uint32_t(v.nx) + 1u, uint32_t(v.ny) + 1u, cx, cy, cz);
-    return fixed_cells_blend(v.cells[c], fx, fy, fz);
-}
-
 // The distance nibble of the brick of cell (cx, cy, cz) (0 without the
 // staged field: nothing is skipped).
 __device__ __forceinline__ uint32_t fixed_brick_distance(const DensityVolume& v, const OccupancyView& occ,

@@ -7,8 +7,8 @@
 // Parallelism in the Construction of BVHs, Octrees, and k-d Trees", HPG
 // 2012): 30-bit Morton codes of the segment centroids, sorted with rocPRIM's
 // radix sort, a binary radix tree over (code, index) -- which bounds its depth
-// by the 62 key bits -- and a bottom-up refit with one arrival counter per
-// node.  The tree that is traversed is cut from it: nodes of up to eight
+// by the 62 key bits -- and boxes that each node forms for itself from unions
+// of 8, 64, 512, ... consecutive leaves.  The tree that is traversed is cut from it: nodes of up to eight
 // children, one octree level each, in 64 bytes.
 //
 // Traversal: one ray per lane, a node's eight boxes per step, children in

@@ -56,13 +56,13 @@ unpack_counts_kernel(const long long* __restrict__ acc, uint32_t* __restrict__ c
 // atomics they are a memory-side line request each, 22 G/s, whatever else the
 // kernel does.  A vertex belongs to one brick of 8x8x8 voxels, so the vertices
 // are counting-sorted by brick instead (a histogram per block, its columns
-// scanned, 8 bytes per vertex written) and a workgroup per brick adds its own
-// in LDS and writes the accumulator and the counts, which then need neither
+// scanned, 8 bytes per vertex written) and workgroups, each of one brick, add them
+// in LDS and write the accumulator and the counts, which then need neither
 // clearing nor unpacking.  The sums are the same integers in any order.
 // 1.77M vertices / 128^3: clearing 8.5, atomics 79.3, unpacking 7.8 us before,
 // now 43.6 (histogram 8.1, columns 4.2, fill 20.5, bricks 10.8; the fill is
 // bound by its scattered writes).
-constexpr uint32_t kBinBricks = 8192;          // a histogram in 32 KB of LDS: up to 160^3
+constexpr uint32_t kBinBricks = 8192;          // a histogram in 32 KB of LDS: up to 160^3 (no larger one was measured)
 constexpr uint32_t kBinBlocks = 256;           // rows of the histogram at most
 constexpr int kBinThreads = 1024, kBrickThreads = 256;
 // A workgroup adds at most this many entries: the further parts of a fuller
