@@ -189,7 +189,7 @@ int vkhr_sort_segments(const float* xyz, uint32_t n_vertices, const uint32_t* in
  * run keeps its pairs in order.  A permutation of the pairs: the volume
  * build's passes then read each strand's vertices contiguously while their
  * workgroups still see few distinct bricks (the one-call build at 136k
- * strands / 256^3: 0.227 ms on the midpoint order, 0.203 ms on this one).
+ * strands / 256^3: 0.216 ms on the midpoint order, 0.183 ms on this one).
  * Same buffers and conditions as vkhr_sort_segments, except that the
  * stream keeps the temporaries (20 bytes per pair) for the next call when
  * they are 256 MB or less. */
