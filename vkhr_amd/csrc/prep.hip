@@ -79,22 +79,36 @@ aabb_final_kernel(const float* __restrict__ partial, int blocks, float* __restri
 // whole lines, where a thread per strand spread every load and store of a
 // wave over 64 strands.  What bounds them is memory: at 136k strands of 13
 // vertices (21 MB in, 21 MB out) the tangents take 13.9 us, 51.4 with a thread
-// per strand; the indices 7.5 us, 12.2 before.  Sixteen lanes whatever the
+// per strand; the indices 7.5 us, 12.2 before; reading the mean first costs
+// the tangents 0.8 (4096 workgroups; 8192 1.3).  Sixteen lanes whatever the
 // strands leave most of them idle on short ones: tangents of
 // 4M strands of two vertices 158 us (56 now), their indices 94 (27).
-constexpr uint32_t kMostLanes = 16, kStrandBlocks = 8192;
+constexpr uint32_t kMostLanes = 16, kStrandBlocks = 4096;
+
+template <uint32_t kLanes, typename Strand>
+__device__ __forceinline__ void grouped_strands(uint32_t n_strands, Strand strand) {
+    const uint32_t lane = threadIdx.x % kLanes, per_block = blockDim.x / kLanes;
+    for (size_t s = size_t(blockIdx.x) * per_block + threadIdx.x / kLanes; s < n_strands;
+         s += size_t(gridDim.x) * per_block)
+        strand(uint32_t(s), lane, kLanes);
+}
 
 // Calls strand(s, lane, lanes) for the strands of this lane's group; a strand
 // has its vertices less `less` items.
 template <typename Strand>
 __device__ __forceinline__ void each_strand(const uint32_t* __restrict__ offsets, uint32_t n_strands, uint32_t less,
                                             Strand strand) {
-    const uint32_t mean = (offsets[n_strands] - offsets[0] - 1u) / n_strands + 1u - less;   // rounded up
-    const uint32_t shift = mean > 8u ? 4u : mean > 4u ? 3u : mean > 2u ? 2u : mean > 1u ? 1u : 0u, lanes = 1u << shift;
-    const uint32_t lane = threadIdx.x & (lanes - 1u), per_block = blockDim.x >> shift;
-    for (size_t s = size_t(blockIdx.x) * per_block + (threadIdx.x >> shift); s < n_strands;
-         s += size_t(gridDim.x) * per_block)
-        strand(uint32_t(s), lane, lanes);
+    const uint64_t n = n_strands, items = offsets[n_strands] - offsets[0] - less * n_strands;
+    if (items > 8u * n)
+        grouped_strands<kMostLanes>(n_strands, strand);
+    else if (items > 4u * n)
+        grouped_strands<8>(n_strands, strand);
+    else if (items > 2u * n)
+        grouped_strands<4>(n_strands, strand);
+    else if (items > n)
+        grouped_strands<2>(n_strands, strand);
+    else
+        grouped_strands<1>(n_strands, strand);
 }
 
 __global__ void __launch_bounds__(256)
