@@ -29,7 +29,7 @@ def test_the_last_tree_is_kept(device, sizes):
         Bvh(styles[n][0], radius[n], styles[n][2])     # built, then destroyed at once
     pairs = styles[sizes[-1]][2].numel() // 2
     assert _given_back() >= 100 * pairs                # a tree is over 128 bytes a pair
-    assert _given_back() <= 0
+    assert _given_back() < 100 * pairs                 # (once)
 
 
 def test_trees_in_turn_are_the_same(device):

@@ -82,7 +82,7 @@ aabb_final_kernel(const float* __restrict__ partial, int blocks, float* __restri
 // per strand; the indices 7.5 us, 12.2 before; reading the mean first costs
 // the tangents 0.8 (4096 workgroups; 8192 1.3).  Sixteen lanes whatever the
 // strands leave most of them idle on short ones: tangents of
-// 4M strands of two vertices 158 us (56 now), their indices 94 (27).
+// 4M strands of two vertices 158 us (58 now), their indices 94 (25).
 constexpr uint32_t kMostLanes = 16, kStrandBlocks = 4096;
 
 template <uint32_t kLanes, typename Strand>
