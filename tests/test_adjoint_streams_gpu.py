@@ -5,6 +5,7 @@ import pytest
 import torch
 
 from tests.test_adjoint_scatter_gpu import DIFF, _scene, _volume
+from vkhr_amd import capi
 from vkhr_amd import device as D
 
 pytestmark = pytest.mark.gpu
@@ -34,3 +35,5 @@ def test_streams_share_the_parameters(device):
     rel = ((shared.double() - want).abs() / (sum(job[-1].abs() for job in jobs) * rounds)).max()
     assert float(rel) <= 7e-5, (shared, want)
     assert np.isfinite(float(rel))
+    for job in jobs:   # (torch hands its streams out again)
+        capi.call("vkhr_release_scratch", job[5].cuda_stream)

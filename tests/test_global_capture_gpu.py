@@ -59,3 +59,4 @@ def test_trees_leave_a_capture_valid(device, mode, kept):
     for tree, w in zip(trees, want):
         for a, b in zip(tree.nodes(), w):
             assert np.array_equal(a, b)
+    capi.call("vkhr_release_scratch", other.cuda_stream)   # (torch hands its streams out again)
