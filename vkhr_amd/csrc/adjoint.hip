@@ -314,6 +314,8 @@ __device__ void scatter_rays_cells(const AdjointArgs& a, CellLds& L, bool active
 // 128^3, 69 MB; 19.5 now, 23.4 with four rows, 20.4 with four levels).
 constexpr int kFoldRows = 2, kFoldLevels = 8;
 
+// kTexels: there are windows' texels.
+template <bool kTexels>
 __global__ void __launch_bounds__(256)
 gather_cells_kernel(const float* __restrict__ cg, const float* __restrict__ texels, float* __restrict__ grad, int nx,
                     int ny, int nz, const double* __restrict__ param_sums, float* __restrict__ d_params) {
@@ -367,9 +369,8 @@ gather_cells_kernel(const float* __restrict__ cg, const float* __restrict__ texe
             for (int r = 0; r < kFoldRows; ++r) {
                 if (x >= nx || y0 + r >= ny) continue;
                 const size_t i = size_t(x) + size_t(nx) * (size_t(y0 + r) + size_t(ny) * size_t(z - 1));
-                float sum = below[r];
-                if (texels) sum += texels[size_t(x) + cx * (size_t(y0 + r) + cy * size_t(z - 1))];
-                grad[i] += sum;
+                const size_t t = size_t(x) + cx * (size_t(y0 + r) + cy * size_t(z - 1));
+                grad[i] += (kTexels ? texels[t] : 0.0f) + below[r];
             }
         }
 #pragma unroll
@@ -777,8 +778,9 @@ extern "C" int vkhr_raymarch_adjoint(const vkhr_volume* volume, const vkhr_camer
     const dim3 fold((volume->nx + kWave - 1) / kWave,
                     (volume->ny + kFoldRows * (256 / kWave) - 1) / (kFoldRows * (256 / kWave)),
                     (volume->nz + kFoldLevels - 1) / kFoldLevels);
-    gather_cells_kernel<<<fold, 256, 0, st>>>(a->cell_grad, a->texel_grad, d_density, int(volume->nx),
-                                              int(volume->ny), int(volume->nz), a->param_sums, d_params);
+    (windows ? gather_cells_kernel<true> : gather_cells_kernel<false>)<<<fold, 256, 0, st>>>(
+        a->cell_grad, a->texel_grad, d_density, int(volume->nx), int(volume->ny), int(volume->nz), a->param_sums,
+        d_params);
     delete a;
     VKHR_CHECK_LAUNCH();
     return VKHR_OK;

@@ -160,45 +160,63 @@ __global__ void __launch_bounds__(kBinThreads) vertex_columns_kernel(VertexBins 
     }
 }
 
-// Every block scans the bricks' totals for itself, which saves a launch
-// (entries in the low half of the words, further parts in the high one).
+// The sum of v over the block's threads before this one.  All of them call it.
+__device__ __forceinline__ uint32_t block_scan(uint32_t* wave_sums, uint32_t v) {
+    const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    uint32_t scan = v;
+    for (int o = 1; o < kWave; o <<= 1) {
+        const uint32_t below = __shfl_up(scan, o, kWave);
+        scan += int(lane) >= o ? below : 0u;
+    }
+    if (lane == kWave - 1) wave_sums[wave] = scan;
+    __syncthreads();
+    uint32_t at = scan - v;
+    for (uint32_t w = 0; w < wave; ++w) at += wave_sums[w];
+    __syncthreads();
+    return at;
+}
+
+// Every block scans the bricks' totals for itself, which saves a launch; the
+// last one, whose vertices are a remainder, writes what the bricks' kernel
+// reads of them.
 __global__ void __launch_bounds__(kBinThreads) vertex_fill_kernel(VertexBins a) {
     extern __shared__ uint32_t cursor[];
-    __shared__ unsigned long long wave_sums[kBinThreads / kWave];
+    __shared__ uint32_t wave_sums[kBinThreads / kWave];
     // the block's share of the bricks in parts (a vertex chunk is under two of n / kBinBlocks: half as many blocks at least)
     __shared__ uint32_t parted[2u * kBinBricks / kBinBlocks], n_parted;
     constexpr uint32_t kPer = kBinBricks / kBinThreads;
     if (threadIdx.x == 0) n_parted = 0u;
-    const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const bool last = blockIdx.x == gridDim.x - 1u;
     for (uint32_t i = threadIdx.x; i < a.n_bricks; i += kBinThreads) cursor[i] = a.total[i];
     __syncthreads();
     const uint32_t per = (a.n_bricks + kBinThreads - 1u) / kBinThreads, i0 = threadIdx.x * per;
-    uint32_t v[kPer];
-    unsigned long long sum = 0;
+    uint32_t v[kPer], sum = 0;
 #pragma unroll
     for (uint32_t c = 0; c < kPer; ++c) {
         v[c] = c < per && i0 + c < a.n_bricks ? cursor[i0 + c] : 0u;
-        sum += v[c] | (unsigned long long)(further_parts(v[c])) << 32;
+        sum += v[c];
     }
-    unsigned long long scan = sum;
-    for (int o = 1; o < kWave; o <<= 1) {
-        const unsigned long long below = __shfl_up(scan, o, kWave);
-        scan += int(lane) >= o ? below : 0ull;
-    }
-    if (lane == kWave - 1) wave_sums[wave] = scan;
-    __syncthreads();
-    unsigned long long at = scan - sum;
-    for (uint32_t w = 0; w < wave; ++w) at += wave_sums[w];
+    uint32_t at = block_scan(wave_sums, sum);
 #pragma unroll
     for (uint32_t c = 0; c < kPer; ++c) {
         if (c < per && i0 + c < a.n_bricks) {
-            cursor[i0 + c] = uint32_t(at);
-            if (blockIdx.x == 0) a.more[i0 + c] = uint32_t(at >> 32);
-            if (further_parts(v[c]) != 0u && (i0 + c) % gridDim.x == blockIdx.x) parted[atomicAdd(&n_parted, 1u)] = i0 + c;
+            cursor[i0 + c] = at;
+            if (v[c] > kPartEntries && (i0 + c) % gridDim.x == blockIdx.x) parted[atomicAdd(&n_parted, 1u)] = i0 + c;
         }
-        at += v[c] | (unsigned long long)(further_parts(v[c])) << 32;
+        at += v[c];
     }
-    if (blockIdx.x == 0 && threadIdx.x == kBinThreads - 1u) a.more[a.n_bricks] = uint32_t(at >> 32);
+    if (last) {   // workgroup-uniform
+        sum = 0;
+#pragma unroll
+        for (uint32_t c = 0; c < kPer; ++c) sum += further_parts(v[c]);
+        at = block_scan(wave_sums, sum);
+#pragma unroll
+        for (uint32_t c = 0; c < kPer; ++c) {
+            if (c < per && i0 + c < a.n_bricks) a.more[i0 + c] = at;
+            at += further_parts(v[c]);
+        }
+        if (threadIdx.x == kBinThreads - 1u) a.more[a.n_bricks] = at;
+    }
     __syncthreads();
     for (uint32_t b = 0; b < n_parted; ++b)
         brick_voxels<kBinThreads>(a, parted[b], [&](uint32_t, size_t voxel) {
@@ -207,10 +225,10 @@ __global__ void __launch_bounds__(kBinThreads) vertex_fill_kernel(VertexBins a) 
         });
     const uint32_t* row = a.hist + size_t(blockIdx.x) * a.n_bricks;
     for (uint32_t i = threadIdx.x; i < a.n_bricks; i += kBinThreads) {
-        if (blockIdx.x == 0) a.start[i] = cursor[i];
+        if (last) a.start[i] = cursor[i];
         cursor[i] += row[i];
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) a.start[a.n_bricks] = a.n_vertices;
+    if (last && threadIdx.x == 0) a.start[a.n_bricks] = a.n_vertices;
     __syncthreads();
     const uint32_t first = blockIdx.x * a.chunk, end = min(first + a.chunk, a.n_vertices);
 #pragma unroll 4
