@@ -46,7 +46,7 @@ batch_raymarch_grid_kernel(BatchDevice d, const RaymarchArgs* __restrict__ args)
 }
 
 // Persistent blocks pulling work items from an atomic queue.  With the pixel
-// body inlined into the loop the compiler allocates 141 registers (3 waves
+// body inlined into the loop the compiler allocates 159 registers (3 waves
 // per SIMD against the grid form's 5); the autotuner measures both.
 __global__ void __launch_bounds__(256)
 batch_raymarch_kernel(BatchDevice d, const RaymarchArgs* __restrict__ args) {

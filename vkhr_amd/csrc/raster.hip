@@ -509,10 +509,11 @@ __device__ void colour_segments(const RasterArgs& a, WaveShared& W, uint32_t s, 
     const uint32_t block_base = block_sums[1];
     Walk w = walk_start(L, 0, 0, a.width, a.height);
     int head = 0, count = 0;  // wave-uniform ring state
-    // Fragments a lane has found ahead of the round that queues them: while some lane looks for its next one the others walk on, so
-    // that a round does not wait for the lane that has furthest to go.  Without
-    // them (each lane at its next fragment every round) the pass takes 993 us
-    // instead of 955 at 136k strands / 1080p; two or four are no better.
+    // Fragments a lane has found ahead of the round that queues them: while
+    // some lane looks for its next one the others walk on, so that a round does
+    // not wait for the lane that has furthest to go.  Without them (each lane at
+    // its next fragment every round) the pass took 993 us where it took 955 at
+    // 136k strands / 1080p (up to 1010 on other cards); two or four are no better.
     constexpr int kAhead = 3;
     uint32_t next_pix[kAhead];
     double next_dp[kAhead];
